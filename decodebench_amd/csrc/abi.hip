@@ -303,6 +303,8 @@ const Knob kKnobs[] = {
      "0 (automatic) or a multiple of 8", nullptr},
     {"gemv_xb", &dbk::Tuning::gemv_xb, [](int v) { return v == 0 || v == 1; }, "0 or 1",
      nullptr},
+    {"gemv_tile", &dbk::Tuning::gemv_tile, [](int v) { return v >= 0 && v <= 2; },
+     "0 (automatic), 1 or 2", nullptr},
     {"f4_launch", &dbk::Tuning::f4_launch, [](int v) { return v >= 0 && v <= 2; },
      "0 (both launches), 1 (split kernel only) or 2 (merge only)", nullptr},
 };

@@ -26,15 +26,18 @@ struct Tuning {
   int f4_line = 0;             // F4 score layout: 0 auto, 1 whole-line K loads, 2 plain
   int f4_combine_groups = 0;   // split groups per F4 merge workgroup (0: auto)
   int f4_depth = 0;            // F4 tiles in flight per wave: 0 auto, 1 or 2
-  int gemv_long_kc = 0;        // streamed-x MFMA GEMV k-steps per chunk: 0 auto, 2 or 4
+  int gemv_long_kc = 0;        // long-row MFMA GEMV k-steps per chunk: 0 auto, 2 or 4
   int gemv_long_gpw = 0;       // long-row MFMA GEMV row groups per workgroup: 0 auto, 1, 2, 4
   int gemv_long_stage = 0;     // long-row MFMA GEMV x: 0 auto, 1 direct, 2 LDS-staged
-  int gemv_pair_min_batch = 0; // gate/up pair rows from which x streams (0: 17)
+  int gemv_pair_min_batch = 0; // gate/up pair rows from which K = 2048 and 4096 take
+                               // gemv_tile (0: 17)
   int stream_waves = 0;        // db_stream_read waves per workgroup: 0 (4), 1, 2 or 4
   int gemv_pass_grid = 0;      // one-matrix MFMA GEMV above 16 rows: workgroups per
                                // 16-row pass (0: CUs / passes; else a multiple of 8)
   int gemv_xb = 0;             // 1: 32-row passes (rows 16..31 of x in LDS) on the
                                // full grid instead
+  int gemv_tile = 0;           // batches of 2 rows and more (gemv_mfma_min_batch if set):
+                               // 0 automatic, 1 gemv_tile, 2 never gemv_tile
   int f4_launch = 0;           // measurement hook for the two-launch F4: 0 both
                                // launches, 1 the split kernel only, 2 the merge only
 };
@@ -84,6 +87,12 @@ hipError_t launch_gemv(GemvMode mode, const void* x, const void* gamma,
 // or e4m3 weights, K in {2048, 4096}.
 bool gemv_mfma_supported(GemvMode mode, int B, int K, int N);
 hipError_t launch_gemv_mfma(GemvMode mode, const void* x, const void* gamma,
+                            const GemvWeights& w, void* y, int B, int K, int N, float eps,
+                            int cu_count, hipStream_t stream);
+
+// Batched GEMV on full 16 x 16 MFMA tiles with streamed activations
+// (gemv_tile.hip): any K the contract allows, any N and batch.
+hipError_t launch_gemv_tile(GemvMode mode, const void* x, const void* gamma,
                             const GemvWeights& w, void* y, int B, int K, int N, float eps,
                             int cu_count, hipStream_t stream);
 

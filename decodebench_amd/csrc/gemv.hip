@@ -4,9 +4,9 @@
 // + SwiGLU pair of the decode-layer chain and the plain projection share one
 // kernel template (gemv_valu.h).  This file instantiates its fp16-weight half
 // and chooses the launch shape; gemv_fp8.hip instantiates the e4m3 half, and
-// batches from 3 rows (2 for the e4m3 norm and gate/up modes and for plain
-// rows longer than 4096) go to the MFMA kernels (gemv_mfma.hip): the
-// crossovers measured on MI355X.
+// batches from 3 rows (2 for the e4m3 norm and gate/up modes, for plain rows
+// longer than 4096 and for large weights of other widths) go to the MFMA
+// kernels (gemv_tile.h, gemv_mfma.hip): the crossovers measured on MI355X.
 #include <mutex>
 #include <unordered_map>
 
@@ -58,6 +58,54 @@ GemvFn gemv_pick_f1_two_rows(int u) {
   }
 }
 
+// Whether a batch of B rows takes the streamed tile kernel (gemv_tile.h)
+// rather than the MFMA kernels of gemv_mfma.hip or the VALU kernel below.
+// The lines lie where the two sides cross, measured on MI355X (graph back to
+// back, interleaved, us, other / tile):
+//  * Widths that gemv_mfma.hip does not take.  The VALU kernel reads the
+//    weights once per pass of 2, 4 or 8 rows and its dot products bound it:
+//    F1 [7168, 5120] at 24 rows 114.8 / 19.4, F1 [5120, 5120] at 4 and 8
+//    rows 15.2 / 12.8 and 33.2 / 12.9.  It stays ahead where one pass does
+//    and the weights are few, so that the tile kernel's LDS staging and
+//    reduction show: [1024, 3072] at 4 rows 4.7 / 5.0, [2048, 1536] at 2
+//    rows 4.1 / 4.7 (2 rows of [8192, 8192] 24.3 / 23.5, F1 27.0 / 23.8).
+//  * The gate/up pair at K = 2048 and 4096, [14336, 4096]: 16-row passes to 16
+//    rows (fp16 40.0 / 39.8 at 16 rows, 38.2 / 39.3 at 4; e4m3 21.4 / 22.4 at
+//    4), the tile kernel above, where the passes read the weights again
+//    (fp16 at 32 and 64 rows 46.7 / 40.9 and 91.0 / 41.1, e4m3 61.9 / 29.4).
+//  * F1 there: registers hold the activations up to 16 rows (fp16 [6144,
+//    4096] 11.3 / 11.5 at 4); above, fp16 takes tiles (24 rows 19.1 / 14.9,
+//    64 rows 28.8 / 21.5) except where one tile per CU leaves the statistic
+//    uncovered ([4096, 4096] at 32 rows 13.1 / 13.6), e4m3 stays (16.9 / 18).
+//  * The plain projection: 3 rows and more (fp16 [4096, 4096] at 8, 24 and
+//    64 rows 8.9 / 8.6, 12.8 / 10.8, 19.8 / 14.6); at K = 2048 only with
+//    more than a tile per CU ([2048, 2048] at 16 rows 5.0 / 5.2); e4m3 with one
+//    tile per CU to 12 rows (6.8 / 6.2 at 8, 7.3 / 7.5 at 16).
+//  * Its rows longer than 4096, above 8 outputs per CU: [4096, 14336] fp16
+//    at 16 rows 28.0 / 25.2, e4m3 at 8 rows 16.0 / 14.8; [1024, 8192] 7.3 /
+//    8.4 stays, and so do one-tile e4m3 calls above 48 rows (33.9 / 35.6).
+bool tile_gemv(GemvMode mode, bool fp8, int B, int K, int N) {
+  const Tuning& t = tuning();
+  if (t.gemv_tile != 0) return t.gemv_tile == 1;
+  const bool pair = gemv_is_swiglu(mode);
+  const long weights = (long)N * K * (pair ? 2 : 1);
+  if (!gemv_mfma_supported(mode, B, K, N)) {
+    if (B == 2) return weights >= 40000000;
+    return B >= 9 || weights >= (B <= 4 ? 10000000 : 4000000);
+  }
+  if (pair) return B >= (t.gemv_pair_min_batch > 0 ? t.gemv_pair_min_batch : 17);
+  const bool one_tile = N <= 4096;
+  if (K > 4096) {
+    const bool forced = t.gemv_long_kc != 0 || t.gemv_long_gpw != 0 || t.gemv_long_stage != 0;
+    return !forced && N > 2048 && !(fp8 && one_tile && B > 48);
+  }
+  if (t.gemv_xb != 0 || t.gemv_pass_grid != 0) return false;
+  if (mode == kGemvRmsNorm)
+    return !fp8 && K == 4096 && B >= 17 && (!one_tile || B <= 24 || B > 32);
+  if (K < 4096) return !one_tile && B >= 3;
+  return fp8 ? (B >= 3 && B <= 12) || (B >= 17 && !one_tile) : B >= 3;
+}
+
 }  // namespace
 
 hipError_t allow_large_lds(const void* fn, size_t dynamic_bytes) {
@@ -84,7 +132,7 @@ hipError_t launch_gemv(GemvMode mode, const void* x, const void* gamma,
                        const GemvWeights& w, void* y, int B, int K, int N, float eps,
                        int cu_count, hipStream_t stream) {
   const int forced_min = tuning().gemv_mfma_min_batch;
-  // At 3 rows the VALU kernel would run two 2-row passes, 1.5-1.8x the MFMA
+  // Where gemv_mfma.hip takes the width.  At 3 rows the VALU kernel would run two 2-row passes, 1.5-1.8x the MFMA
   // time.  At 2 rows (graph back-to-back, us, VALU / MFMA) MFMA takes the
   // e4m3 modes with a norm or two matrices (F1 [4096, 4096] 5.87 / 5.46,
   // F1-QKV 7.17 / 6.81, gate/up pair 22.4 / 19.2, RMSNorm -> gate/up 23.2 /
@@ -96,6 +144,8 @@ hipError_t launch_gemv(GemvMode mode, const void* x, const void* gamma,
   const bool mfma_at_two = (w.fp8 && mode != kGemvPlain) || (mode == kGemvPlain && K > 4096);
   const int auto_min = mfma_at_two ? 2 : 3;
   const int mfma_min = forced_min > 0 ? forced_min : auto_min;
+  if (B >= (forced_min > 0 ? forced_min : 2) && tile_gemv(mode, w.fp8, B, K, N))
+    return launch_gemv_tile(mode, x, gamma, w, y, B, K, N, eps, cu_count, stream);
   if (B >= mfma_min && gemv_mfma_supported(mode, B, K, N))
     return launch_gemv_mfma(mode, x, gamma, w, y, B, K, N, eps, cu_count, stream);
   GemvArgs a;

@@ -1,7 +1,7 @@
-// gemv_mfma.hip -- batched decode GEMV on MFMA for gfx950: gemv_mfma_kernel
-// (passes of 16 or 32 batch rows), and the kernels that also stream the
-// activations, gemv_mfma_long_kernel (rows longer than 4096) and
-// gemv_mfma_tile16_kernel (the gate/up pair above 16 rows).
+// gemv_mfma.hip -- batched decode GEMV on MFMA for gfx950 with the activations
+// in registers, K in {2048, 4096}: gemv_mfma_kernel (passes of 16 or 32 batch
+// rows); and gemv_mfma_long_kernel, which streams them too (few output rows
+// longer than 4096).  gemv_tile.h takes every other batched shape.
 //
 // y[B,N] = op(x[B,K]) . W^T for the four GEMV modes of gemv.hip (plain,
 // RMSNorm-fused F1, gate/up + SwiGLU F2, RMSNorm -> gate/up + SwiGLU) with
@@ -42,10 +42,8 @@
 // matrix the passes of a row group run on one XCD at the same time, so the
 // later passes read its weights from L2 (see launch_gemv_mfma); 32-row
 // passes with rows 16..31 of x in LDS (XB) remain as a tuning option.
-// Plain GEMV with longer rows (K a multiple of 2048 above 4096, the down
-// projection) and the gate/up pair above 16 rows, with or without the
-// RMSNorm, take kernels that stream x as well: gemv_mfma_long_kernel and
-// gemv_mfma_tile16_kernel (below).
+// Plain GEMV of few, longer rows (K a multiple of 2048 above 4096) takes
+// gemv_mfma_long_kernel (below), which streams x as well.
 #include "gemv_valu.h"
 
 namespace dbk {
@@ -773,266 +771,6 @@ __global__ __launch_bounds__(kThreadsM) void gemv_mfma_long_kernel(MfmaArgs a) {
   }
 }
 
-// ---- streamed activations on full 16-row tiles ----------------------------
-// The kernel above spends three quarters of every accumulator: an 8-row
-// group over two half slices fills one v_mfma_f32_16x16x32_f16, but only
-// its two diagonal 8 x 8 blocks are dot products.  For the gate/up pair at
-// 32 rows that would be 7 groups x 2 matrices x 4 tiles of accumulators
-// (224 registers) on a CU's 56 rows; a version built that way had the
-// register allocator move accumulators through a shared temporary between
-// MFMAs and ran 1.6x slower (e4m3).  Here an MFMA
-// takes 16 weight rows (two of the workgroup's 8-row groups) against 16
-// batch rows over the same 32 columns, and every element of D is an output:
-// A row m = row m & 7 of group 2j + (m >> 3), k-group g4 = columns
-// 32 s + 8 g4 of k-step s (fp16) or, for e4m3, columns 64 (s >> 1) +
-// 16 g4 + 8 (s & 1); B column n = batch row 16 bt + n over the same columns.
-// Loading those A operands directly would read 16 rows x 64 bytes (half
-// lines) per instruction.  Instead each 8-row group is loaded as above --
-// lane (g4, h, r8) takes row r8, half h of a 128-byte line, 8 whole lines
-// per instruction -- and the two groups of a tile are merged into its A
-// operands with one DPP row_ror:8 move per register: lanes 8..15 of each
-// 16-lane row of the first group's register take lanes 0..7 of the
-// second's (the tile's half-0 operand), and lanes 0..7 of the second's take
-// lanes 8..15 of the first's (its half-1 operand).
-// Waves own K / WV slices as above and walk them in chunks of KC k-steps;
-// accumulators stay in registers; the K-slice partial sums meet in LDS with
-// the same layout and epilogue as above.  A workgroup owns up to 2 T
-// groups; a last tile with one group duplicates it in rows 8..15, which are
-// not stored.  Launched with N a multiple of 8 and 2 N K bytes below 4 GiB
-// (32-bit lane offsets; every row of a live group below N).
-// NORM (RMSNorm -> gate/up, K <= 4096): before the stream each wave sums x^2
-// over its slice for every batch row of the pass; each streamed x chunk is
-// then normalised as fp16(fp16(x * inv_rms) * gamma).
-__device__ __forceinline__ u4 tile_half0(const u4& g0, const u4& g1) {
-  u4 t;
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-    t[i] = (unsigned)__builtin_amdgcn_update_dpp((int)g0[i], (int)g1[i], kRowRor8, 0xf, 0xc,
-                                                 false);
-  return t;
-}
-__device__ __forceinline__ u4 tile_half1(const u4& g0, const u4& g1) {
-  u4 t;
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-    t[i] = (unsigned)__builtin_amdgcn_update_dpp((int)g1[i], (int)g0[i], kRowRor8, 0xf, 0x3,
-                                                 false);
-  return t;
-}
-
-template <int NWM, int WV, int KC, int BT16, int T, bool FP8, bool NORM>
-__global__ __launch_bounds__(WV * kWave) void gemv_mfma_tile16_kernel(MfmaArgs a) {
-  constexpr int kThreads = WV * kWave;
-  constexpr int kStepsPerLoad = FP8 ? 2 : 1;  // k-steps in a 16-byte A operand
-  constexpr int LS = 2 * kStepsPerLoad;       // k-steps per line load (both halves)
-  static_assert(KC % LS == 0, "a chunk holds whole lines");
-  constexpr int KWC = KC / LS;                // line loads per group and chunk
-  constexpr int NG = 2 * T;                   // 8-row groups
-  constexpr int kPass = 16 * BT16;
-  constexpr int kXL = BT16 * KC;
-  static_assert((WV & (WV - 1)) == 0, "waves per workgroup: a power of 2");
-  extern __shared__ __align__(16) unsigned char dyn_lds[];
-  float* const part = reinterpret_cast<float*>(dyn_lds);  // [2T][NWM][WV][kPass][8]
-
-  const int lane = threadIdx.x & (kWave - 1);
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  const int c16 = lane & 15;
-  const int g4 = lane >> 4;
-  const int bx = blockIdx.x;
-  const int grid = gridDim.x;
-  const int b0 = blockIdx.y * kPass;
-  const int nb = min(kPass, a.B - b0);
-  const int slice = a.K / WV;
-  const int nch = slice / (32 * KC);  // chunks of KC k-steps of 32 columns
-  const int sbase = ((wave + bx + (bx >> 3)) & (WV - 1)) * slice;
-  const int xcol0 = sbase + (FP8 ? 16 * g4 : 8 * g4);
-  const int my_groups = min(a.gpw, (a.groups - bx + grid - 1) / grid);
-  const int esz = FP8 ? 1 : 2;
-  const unsigned char* wmat[2] = {static_cast<const unsigned char*>(a.w0),
-                                  static_cast<const unsigned char*>(a.w1)};
-
-  // Weight lane offset: row r8 of the group, half h of the line; groups are
-  // gstride apart (group q of the workgroup is bx + grid q).
-  const int r8 = c16 & 7;
-  const int half = c16 >> 3;
-  const int wcol0 = sbase + (FP8 ? 64 * half + 16 * g4 : 32 * half + 8 * g4);
-  const unsigned woff = ((unsigned)(bx * kRowsPerGroup + r8) * (unsigned)a.K +
-                         (unsigned)wcol0) * esz;
-  const size_t gstride = (size_t)grid * kRowsPerGroup * a.K * esz;
-  const _Float16* xp[BT16];
-#pragma unroll
-  for (int bt = 0; bt < BT16; ++bt)
-    xp[bt] = a.x + (size_t)(b0 + min(16 * bt + c16, nb - 1)) * a.K + xcol0;
-  // Column offset of line load p within a chunk, and of k-step t's
-  // activations.
-  auto wcol = [](int p) { return (FP8 ? 128 : 64) * p; };
-  auto xcol = [](int t) { return FP8 ? 64 * (t >> 1) + 8 * (t & 1) : 32 * t; };
-
-  // NORM: gamma at the activations' columns, loaded with each chunk.
-  constexpr int kGL = NORM ? KC : 1;
-  auto load = [&](u4 (&xs)[kXL], u4 (&gs)[kGL], u4 (&ws)[NG][NWM][KWC], int c) {
-    const int c0 = 32 * KC * c;
-#pragma unroll
-    for (int j = 0; j < NG; ++j) {
-      // Groups past the workgroup's last re-read that one (rows not stored).
-      const size_t goff = gstride * min(j, my_groups - 1);
-#pragma unroll
-      for (int m = 0; m < NWM; ++m)
-#pragma unroll
-        for (int p = 0; p < KWC; ++p)
-          ws[j][m][p] = ld_stream(wmat[m] + goff + (size_t)(c0 + wcol(p)) * esz + woff);
-    }
-#pragma unroll
-    for (int i = 0; i < kXL; ++i) xs[i] = ld16(xp[i / KC] + c0 + xcol(i % KC));
-    if constexpr (NORM) {
-#pragma unroll
-      for (int t = 0; t < KC; ++t) gs[t] = ld16(a.gamma + xcol0 + c0 + xcol(t));
-    }
-  };
-  f4 acc[T][NWM][BT16];
-#pragma unroll
-  for (int j = 0; j < T; ++j)
-#pragma unroll
-    for (int m = 0; m < NWM; ++m)
-#pragma unroll
-      for (int bt = 0; bt < BT16; ++bt) acc[j][m][bt] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-  // A operand u (16 bytes, kStepsPerLoad k-steps from k-step t0) of tile j.
-  auto mma = [&](const u4& u, int j, int m, int t0, const u4 (&xs)[kXL]) {
-    u4 av[kStepsPerLoad];
-    if constexpr (FP8) e4m3x16_to_h(u, av[0], av[1]);
-    else av[0] = u;
-#pragma unroll
-    for (int s = 0; s < kStepsPerLoad; ++s)
-#pragma unroll
-      for (int bt = 0; bt < BT16; ++bt)
-        acc[j][m][bt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-            __builtin_bit_cast(h8, av[s]), __builtin_bit_cast(h8, xs[bt * KC + t0 + s]),
-            acc[j][m][bt], 0, 0, 0);
-  };
-  float inv[BT16];  // NORM: 1 / rms of this lane's batch rows
-  auto consume = [&](const u4 (&xl)[kXL], const u4 (&gs)[kGL], const u4 (&ws)[NG][NWM][KWC]) {
-    // NORM: fp16(fp16(x * inv_rms) * gamma), the torch stage's rounding
-    // points (see norm_mul).
-    u4 xs[kXL];
-#pragma unroll
-    for (int i = 0; i < kXL; ++i) xs[i] = NORM ? norm_mul(xl[i], gs[i % KC], inv[i / KC]) : xl[i];
-#pragma unroll
-    for (int p = 0; p < KWC; ++p)
-#pragma unroll
-      for (int j = 0; j < T; ++j)
-#pragma unroll
-        for (int m = 0; m < NWM; ++m) {
-          const u4& g0 = ws[2 * j][m][p];
-          const u4& g1 = ws[2 * j + 1][m][p];
-          mma(tile_half0(g0, g1), j, m, LS * p, xs);
-          mma(tile_half1(g0, g1), j, m, LS * p + kStepsPerLoad, xs);
-        }
-  };
-
-  u4 xa[kXL], ga[kGL], wa[NG][NWM][KWC], xb[kXL], gb[kGL], wb[NG][NWM][KWC];
-  load(xa, ga, wa, 0);  // in flight during the statistic below
-  if constexpr (NORM) {
-    // x^2 over this wave's K slice for every batch row of the pass, 8 rows
-    // at a time (lane l takes 16-byte pieces l and l + 64 of a row's slice,
-    // which covers K <= 4096), then over the waves in LDS.
-    __shared__ float red[WV][kPass];
-    const int pieces = slice / 8;
-    const u4 zero4 = {0, 0, 0, 0};
-    for (int r0 = 0; r0 < nb; r0 += 8) {
-      u4 v[8][2];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const _Float16* xr = a.x + (size_t)(b0 + min(r0 + i, nb - 1)) * a.K + sbase;
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-          v[i][h] = lane + 64 * h < pieces ? ld16(xr + 8 * (lane + 64 * h)) : zero4;
-      }
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const float ss = wave_sum(dot8(v[i][1], v[i][1], dot8(v[i][0], v[i][0], 0.0f)));
-        if (lane == 0 && r0 + i < nb) red[wave][r0 + i] = ss;
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int bt = 0; bt < BT16; ++bt) {
-      const int r = min(16 * bt + c16, nb - 1);
-      float tot = 0.0f;
-#pragma unroll
-      for (int w = 0; w < WV; ++w) tot += red[w][r];
-      inv[bt] = 1.0f / sqrtf(tot / (float)a.K + a.eps);
-    }
-  }
-  int c = 0;
-  // A scheduling barrier after each load keeps the next chunk in flight
-  // while the current one is consumed (otherwise the compiler sinks the
-  // loads below the current chunk's waits), and the tail is straight-line
-  // code per case.  Measured at [14336, 4096], 17-32 rows (µs): fp16 pair
-  // 39.7 -> 39.2 (B = 17), 42.1 -> 41.8 (B = 32); RMSNorm -> gate/up 46.4
-  // -> 44.8, 50.3 -> 48.9; e4m3 pair 27.9 -> 27.4 (B = 32), RMSNorm ->
-  // gate/up 32.6 -> 31.3, 36.3 -> 34.8.
-  for (; c + 3 <= nch; c += 2) {
-    load(xb, gb, wb, c + 1);
-    __builtin_amdgcn_sched_barrier(0);
-    consume(xa, ga, wa);
-    load(xa, ga, wa, c + 2);
-    __builtin_amdgcn_sched_barrier(0);
-    consume(xb, gb, wb);
-  }
-  if (c + 1 < nch) {
-    load(xb, gb, wb, c + 1);
-    __builtin_amdgcn_sched_barrier(0);
-    consume(xa, ga, wa);
-    consume(xb, gb, wb);
-  } else {
-    consume(xa, ga, wa);
-  }
-
-  // D[4 g4 + i][c16] = tile row 4 g4 + i (group 2j + (g4 >> 1), row
-  // 4 (g4 & 1) + i) against batch row 16 bt + c16.
-  auto slot = [&](int q, int m, int v, int n) {
-    return part + ((((q * NWM + m) * WV + v) * kPass + n) * kRowsPerGroup);
-  };
-#pragma unroll
-  for (int j = 0; j < T; ++j) {
-    const int q = 2 * j + (g4 >> 1);
-    if (q < my_groups) {
-#pragma unroll
-      for (int m = 0; m < NWM; ++m)
-#pragma unroll
-        for (int bt = 0; bt < BT16; ++bt)
-          *reinterpret_cast<f4*>(slot(q, m, wave, 16 * bt + c16) + 4 * (g4 & 1)) =
-              acc[j][m][bt];
-    }
-  }
-  __syncthreads();
-
-  for (int idx = threadIdx.x; idx < my_groups * kPass * kRowsPerGroup; idx += kThreads) {
-    const int q = idx / (kPass * kRowsPerGroup);
-    const int n = (idx / kRowsPerGroup) % kPass;
-    const int r = idx % kRowsPerGroup;
-    const int row = (bx + grid * q) * kRowsPerGroup + r;
-    if (n >= nb) continue;
-    float s0 = 0.0f, s1 = 0.0f;
-#pragma unroll
-    for (int v = 0; v < WV; ++v) {
-      s0 += slot(q, 0, v, n)[r];
-      if constexpr (NWM == 2) s1 += slot(q, NWM - 1, v, n)[r];
-    }
-    if constexpr (FP8) {
-      s0 *= a.s0[row];
-      if constexpr (NWM == 2) s1 *= a.s1[row];
-    }
-    float out = s0;
-    if constexpr (NWM == 2) {
-      const float gq = (float)to_h(s0);
-      const float uq = (float)to_h(s1);
-      out = (float)to_h(gemv_silu(gq)) * uq;
-    }
-    a.y[(size_t)(b0 + n) * a.N + row] = to_h(out);
-  }
-}
-
 using MfmaFn = void (*)(MfmaArgs);
 
 // One group per register set, two sets alternating (load set B, consume A,
@@ -1100,38 +838,6 @@ MfmaFn pick_long(int kc, int bt, int gpw, bool xs) {
   return xs ? pick_long_kc<FP8, true>(kc, bt, gpw) : pick_long_kc<FP8, false>(kc, bt, gpw);
 }
 
-// The gate/up pair on 16-row tiles: 4 waves, 2 (fp16) or 4 (e4m3, whose
-// whole lines span 4 k-steps) k-steps per chunk, 16 or 32 batch rows, 1, 2
-// or 4 tiles (2, 4 or 8 groups).
-constexpr int kPairWaves = 4;
-
-template <int KC, int BT16, bool FP8, bool NORM>
-MfmaFn pick_pair_t(int t) {
-  return t == 1 ? gemv_mfma_tile16_kernel<2, kPairWaves, KC, BT16, 1, FP8, NORM>
-         : t == 2 ? gemv_mfma_tile16_kernel<2, kPairWaves, KC, BT16, 2, FP8, NORM>
-                  : gemv_mfma_tile16_kernel<2, kPairWaves, KC, BT16, 4, FP8, NORM>;
-}
-
-// fp16 with the norm takes 2-k-step chunks only (4 would spill at 32 rows).
-template <bool FP8, bool NORM>
-MfmaFn pick_pair_n(int kc, int bt16, int t) {
-  if constexpr (!FP8 && NORM) {
-    (void)kc;
-    return bt16 == 1 ? pick_pair_t<2, 1, FP8, NORM>(t) : pick_pair_t<2, 2, FP8, NORM>(t);
-  } else {
-    if constexpr (!FP8) {
-      if (kc == 2)
-        return bt16 == 1 ? pick_pair_t<2, 1, FP8, NORM>(t) : pick_pair_t<2, 2, FP8, NORM>(t);
-    }
-    return bt16 == 1 ? pick_pair_t<4, 1, FP8, NORM>(t) : pick_pair_t<4, 2, FP8, NORM>(t);
-  }
-}
-
-template <bool FP8>
-MfmaFn pick_pair(int kc, int bt16, int t, bool norm) {
-  return norm ? pick_pair_n<FP8, true>(kc, bt16, t) : pick_pair_n<FP8, false>(kc, bt16, t);
-}
-
 }  // namespace
 
 // Long rows (plain GEMV, K a multiple of 2048 above 4096): both operands
@@ -1140,19 +846,9 @@ static bool long_rows(GemvMode mode, int K) {
   return mode == kGemvPlain && K > 4096 && K % 2048 == 0;
 }
 
-// The gate/up pair from pair_min rows (K a multiple of 2048, N of 8): x
-// streams, one pass up to 32 rows.
-static bool pair_rows(GemvMode mode, int B, int K, int N) {
-  const int pair_min = tuning().gemv_pair_min_batch > 0 ? tuning().gemv_pair_min_batch : 17;
-  // The RMSNorm mode's statistic pass covers K <= 4096 (2 pieces per lane).
-  const bool mode_ok = mode == kGemvSwiGLU || (mode == kGemvRmsNormSwiGLU && K <= 4096);
-  return mode_ok && K % 2048 == 0 && N % kRowsPerGroup == 0 &&
-         (size_t)2 * N * K * 2 < ((size_t)1 << 32) && B >= pair_min;
-}
-
 bool gemv_mfma_supported(GemvMode mode, int B, int K, int N) {
   if (B < 2 || N < 1) return false;
-  if (long_rows(mode, K) || pair_rows(mode, B, K, N)) return true;
+  if (long_rows(mode, K)) return true;
   if (K != 2048 && K != 4096) return false;  // K / 512 = 4 or 8 k-steps per half
   const int groups = (N + kRowsPerGroup - 1) / kRowsPerGroup;
   return groups <= 256 * kMaxGroupsPerWg;
@@ -1205,41 +901,6 @@ static hipError_t launch_gemv_mfma_long(const MfmaArgs& a0, bool fp8, int cu_cou
   return hipGetLastError();
 }
 
-// The gate/up pair from 17 rows, measured at [14336, 4096] (µs, graph back to
-// back; 16-row passes / streamed on 8-row halves / on 16-row tiles loaded
-// directly / on 16-row tiles merged from whole lines): fp16 B = 17 74.1 /
-// 43.5 / 53.0 / 39.7, B = 32 76.2 / 44.4 / 55.1 / 42.0; e4m3 B = 17 40.5 /
-// 43.7 / 29.3 / 25.5, B = 32 42.4 / 45.3 / 32.0 / 28.1.  The halves hold
-// four times the accumulators (the register allocator then moved them
-// through a shared temporary between MFMAs); the direct tiles read half
-// lines.  4-k-step fp16 chunks measured 1.5-2.3 us slower, 8-wave
-// workgroups 5-6 us slower.
-static hipError_t launch_gemv_mfma_pair(const MfmaArgs& a0, bool norm, bool fp8, int cu_count,
-                                        hipStream_t stream) {
-  MfmaArgs a = a0;
-  // The kernel's 32-bit lane offsets (see gemv_mfma_tile16_kernel).
-  if (a.N % kRowsPerGroup != 0 ||
-      (size_t)2 * a.N * a.K * (fp8 ? 1 : 2) >= ((size_t)1 << 32))
-    return hipErrorInvalidValue;
-  const int bt16 = a.B <= 16 ? 1 : 2;  // passes of 16 or 32 rows
-  const int kc = fp8 ? 4 : !norm && tuning().gemv_long_kc == 4 ? 4 : 2;
-  int gpw = (a.groups + cu_count - 1) / cu_count;
-  if (gpw > 8) gpw = 8;
-  const int t = gpw <= 2 ? 1 : gpw <= 4 ? 2 : 4;
-  a.gpw = gpw;
-  const int grid = (a.groups + gpw - 1) / gpw;
-  const MfmaFn fn =
-      fp8 ? pick_pair<true>(kc, bt16, t, norm) : pick_pair<false>(kc, bt16, t, norm);
-  const size_t lds = sizeof(float) * 2 * t * 2 * kPairWaves * 16 * bt16 * kRowsPerGroup;
-  if (lds > 48 * 1024) {
-    hipError_t e = allow_large_lds(reinterpret_cast<const void*>(fn), lds);
-    if (e != hipSuccess) return e;
-  }
-  dim3 g(grid, (a.B + 16 * bt16 - 1) / (16 * bt16));
-  hipLaunchKernelGGL(fn, g, dim3(kPairWaves * kWave), lds, stream, a);
-  return hipGetLastError();
-}
-
 hipError_t launch_gemv_mfma(GemvMode mode, const void* x, const void* gamma,
                             const GemvWeights& w, void* y, int B, int K, int N, float eps,
                             int cu_count, hipStream_t stream) {
@@ -1258,8 +919,6 @@ hipError_t launch_gemv_mfma(GemvMode mode, const void* x, const void* gamma,
   a.eps = eps;
   a.groups = (N + kRowsPerGroup - 1) / kRowsPerGroup;
   if (long_rows(mode, K)) return launch_gemv_mfma_long(a, w.fp8, cu_count, stream);
-  if (pair_rows(mode, B, K, N))
-    return launch_gemv_mfma_pair(a, mode == kGemvRmsNormSwiGLU, w.fp8, cu_count, stream);
   const int kh = K / 512;
   const int nwm = gemv_is_swiglu(mode) ? 2 : 1;
   // One weight matrix above 16 rows: P = ceil(B / 16) passes of 16 rows

@@ -36,14 +36,18 @@ extern "C" {
  *                         workgroup: 1, 2, 4 or 8; 0 automatic)
  *  "f4_depth"            (tiles in flight per wave of the 8-wave whole-line F4
  *                         kernel: 1 or 2; 0 automatic)
- *  "gemv_long_kc"        (k-steps of 32 columns per chunk of the MFMA GEMVs
- *                         that stream their activations: 2 or 4; 0 automatic)
- *  "gemv_long_gpw"       (8-row groups per workgroup of the long-row kernel:
- *                         1, 2 or 4; 0 automatic)
+ *  "gemv_long_kc"        (k-steps of 32 columns per chunk of the long-row
+ *                         MFMA GEMV: 2 or 4; 0 automatic)
+ *  "gemv_long_gpw"       (its 8-row groups per workgroup: 1, 2 or 4; 0
+ *                         automatic)
  *  "gemv_long_stage"     (its activations: 1 loaded as B operands, 2 staged
- *                         through LDS; 0 automatic)
- *  "gemv_pair_min_batch" (batch rows from which the gate/up pair streams its
- *                         activations; 0 automatic, 17)
+ *                         through LDS; 0 automatic).  Any of these three set
+ *                         keeps plain rows longer than 4096 on that kernel
+ *  "gemv_pair_min_batch" (batch rows from which the gate/up pair at K = 2048
+ *                         and 4096 streams its activations on 16 x 16 tiles;
+ *                         0 automatic, 17)
+ *  "gemv_tile"           (batches of 2 rows and more: 1 always the streamed
+ *                         16 x 16 tile kernel, 2 never; 0 automatic)
  *  "stream_waves"        (db_stream_read's waves per workgroup: 1, 2 or 4; 0
  *                         is 4)
  *  "gemv_pass_grid"      (one weight matrix above 16 batch rows on MFMA:
@@ -51,7 +55,8 @@ extern "C" {
  *                         automatic)
  *  "gemv_xb"             (1: 32-row passes with rows 16..31 of the
  *                         activations in LDS on the full grid; 0, the default,
- *                         off)
+ *                         off).  Either of these two set keeps one matrix at
+ *                         K = 2048 and 4096 off the tile kernel
  *  "f4_launch"           (a call of F4 whose split merge runs in a second
  *                         launch makes only one of its two launches: 1 the
  *                         split kernel, 2 the merge, which then reads whatever

@@ -1,0 +1,147 @@
+"""The streamed tile GEMV (gemv_tile) at the edges of its tiles.
+
+Every case forces the kernel and compares with fp64 products of the same
+fp16 inputs.  The bound is derived per output, from the fp16 roundings
+(2^-11 each) and the fp32 sums:
+
+* one matrix: 2^-11 |y| for the output, (2^-11 + K 2^-23) sum_k |w p| for the
+  rounded operands (norm modes) and the sums;
+* gate/up: that error on gate and up, their own fp16 rounding, carried through
+  silu(g) u (|silu'| <= 1.1), and the roundings of silu and of the product.
+"""
+
+import pytest
+
+torch = pytest.importorskip("torch")
+
+from decodebench_amd import ops  # noqa: E402
+from decodebench_amd.quant import dequantize_e4m3_rows, quantize_e4m3_rows  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+U = 2.0 ** -11   # fp16 rounding
+TINY = 2.0 ** -24
+
+
+@pytest.fixture(autouse=True)
+def _force_tile():
+    ops.tune("gemv_tile", 1)
+    yield
+    ops.tune("gemv_tile", 0)
+
+
+def _randn(gen, *shape, std=1.0, mean=0.0):
+    t = torch.randn(*shape, generator=gen, device="cuda", dtype=torch.float32)
+    return (t * std + mean).half()
+
+
+def _call(mode, x, g, W, s):
+    if mode == "gemv":
+        return ops.gemv(x, W[0], w_scale=s[0])
+    if mode == "f1":
+        return ops.f1_rmsnorm_gemv(x, g, W[0], w_scale=s[0])
+    if mode == "f2":
+        return ops.f2_gateup_swiglu(x, W[0], W[1], s[0], s[1])
+    return ops.f2_rmsnorm_gateup_swiglu(x, g, W[0], W[1], sg=s[0], su=s[1])
+
+
+def _check(mode, x, g, W, s, W64):
+    norm = mode in ("f1", "f2n")
+    K = x.shape[1]
+    p = x.double()
+    if norm:
+        p = p * torch.rsqrt(p.square().mean(-1, keepdim=True) + 1e-6) * g.double()
+
+    def linear(w):
+        wt = w.t().contiguous()
+        return p @ wt, ((U if norm else 0.0) + K * 2.0 ** -23) * (p.abs() @ wt.abs())
+
+    y = _call(mode, x, g, W, s).double()
+    a, da = linear(W64[0])
+    if mode in ("gemv", "f1"):
+        ref, bound = a, da + U * a.abs()
+    else:
+        u, du = linear(W64[1])
+        da, du = da + U * a.abs(), du + U * u.abs()
+        sil = a * torch.sigmoid(a)
+        ref = sil * u
+        bound = 1.1 * da * (u.abs() + du) + sil.abs() * du + 3 * U * ref.abs()
+    # 1.01: the bound's own second-order terms
+    bad = (y - ref).abs() > 1.01 * bound + 2 * TINY
+    assert torch.isfinite(y).all()
+    assert not bad.any(), f"{int(bad.sum())} outputs outside the bound, worst " \
+                          f"{((y - ref).abs() / (bound + TINY)).max().item():.2f} of it"
+
+
+def _weights(gen, n, N, K, dtype):
+    W, s, W64 = [], [], []
+    for _ in range(n):
+        w = _randn(gen, N, K, std=K ** -0.5)
+        if dtype == "fp8":
+            w, sc = quantize_e4m3_rows(w)
+            W64.append(dequantize_e4m3_rows(w, sc).double())
+        else:
+            sc = None
+            W64.append(w.double())
+        W.append(w)
+        s.append(sc)
+    return W, s, W64
+
+
+# Batch rows at the edges of the 8-row groups and the 64-row pass; K below one
+# block, at its edges and with 1 to 9 blocks per wave; N at the edges of the
+# 4-row shares and of every tile count (256 workgroups x 16 rows, 8 outputs for
+# the pair), and above what 8 tiles hold.
+CASES = [
+    ("gemv", "f16", 2, 8, 1), ("f1", "f16", 3, 16, 3), ("f2", "f16", 9, 64, 5),
+    ("f2n", "f16", 16, 72, 1023), ("gemv", "fp8", 7, 16, 1), ("f1", "fp8", 8, 128, 1025),
+    ("f2", "fp8", 17, 144, 4), ("f2n", "fp8", 24, 112, 1030),
+    ("gemv", "f16", 25, 3000, 2052), ("f1", "f16", 32, 2568, 4097), ("f1", "fp8", 33, 2576, 4095),
+    ("gemv", "fp8", 48, 4608, 1500), ("f2", "f16", 49, 1000, 2049), ("f2n", "fp8", 64, 1040, 2047),
+    ("f1", "f16", 65, 520, 515), ("gemv", "fp8", 130, 528, 4100),
+    ("gemv", "f16", 5, 200, 28673), ("gemv", "f16", 64, 136, 20481), ("f1", "fp8", 41, 272, 24577),
+    ("gemv", "f16", 12, 64, 33000), ("f2", "f16", 6, 328, 14337), ("f2", "fp8", 64, 192, 12289),
+    ("f2n", "f16", 40, 264, 10241), ("f2n", "fp8", 4, 272, 8193), ("f2", "f16", 20, 64, 16500),
+]
+
+
+@pytest.mark.parametrize("mode,dtype,B,K,N", CASES)
+def test_tile_edges(mode, dtype, B, K, N):
+    print(f"[tile] {mode} {dtype} B={B} K={K} N={N}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(B * 7919 + K + N)
+    x = _randn(gen, B, K)
+    g = _randn(gen, K, std=0.1, mean=1.0)
+    _check(mode, x, g, *_weights(gen, 2 if mode in ("f2", "f2n") else 1, N, K, dtype))
+
+
+@pytest.mark.parametrize("dtype", ["f16", "fp8"])
+@pytest.mark.parametrize("rows", ["tiny", "large", "mixed", "late", "early", "zero"])
+def test_tile_norm_keeps_precision_over_the_fp16_range(rows, dtype):
+    """x whose products with gamma leave fp16 (tiny, large, a row of each), or
+    whose first columns do not say so (late: 3e4 after columns of 1e-3; early:
+    the other way round), and rows of zeros."""
+    print(f"[tile-norm] {rows} {dtype}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    B, K, N = 12, 1536, 300
+    # a few ulps wide, so that tiny values keep their relative precision
+    x = (_randn(gen, B, K).sign().float() * (1 + 0.5 * torch.rand(B, K, generator=gen,
+                                                                  device="cuda")))
+    scale = torch.ones(B, K, device="cuda")
+    if rows == "tiny":
+        scale *= 2.0 ** -13
+    elif rows == "large":
+        scale *= 2.0 ** 14
+    elif rows == "mixed":
+        scale[::2] *= 2.0 ** -12
+        scale[1::2] *= 2.0 ** 14
+    elif rows == "late":
+        scale *= 2.0 ** -10
+        scale[:, K // 2:] = 2.0 ** 14
+    elif rows == "early":
+        scale *= 2.0 ** 14
+        scale[:, K // 2:] = 2.0 ** -3
+    x = (x * scale).half()
+    if rows == "zero":
+        x[3:9] = 0
+    g = _randn(gen, K, std=1.0, mean=16.0)
+    _check("f1", x, g, *_weights(gen, 1, N, K, dtype))
