@@ -775,16 +775,68 @@ size_t f4_workspace_bytes(int B, int Hq, int Hkv, int S, int D) {
          pairs * S * G * D * sizeof(float);
 }
 
+// Split count of a call: the one whose estimated time is least.  The chip
+// works through ceil(pairs S / CUs) rounds of workgroups, each as long as its
+// longest split: about 0.3 us per 16-row tile while the whole chip streams,
+// 1.6 us more per further round, and the merge (1.5 us to 8 splits, which one
+// thread per output merges, 2.9 us above, 3.5 where 4 waves take a second
+// chunk of splits).  So a count that just spills over
+// into another round is avoided (20 x 8 pairs at L = 3001 with 2 splits, 1.25
+// rounds, 54.7 us; with 3, 1.9 rounds, 43.9), and so is one round of few
+// workgroups (12 x 8 pairs: 3 splits 40.7, 2 splits 34.4, 5 splits 31.2).
+// Measured on MI355X (graph back to back, us, a workgroup per CU rounded up /
+// by this estimate): B = 3, 5, 7 at L = 12000, 9000, 4000 40.4 / 30.5, 48.6 /
+// 33.8, 32.9 / 24.7; B = 10, 24, 36, 40 at L = 3001 30.8 / 24.8, 61.9 / 50.6,
+// 103.8 / 79.9, 106.2 / 82.9; B = 1 at L = 300 and 3001 6.4 / 5.3, 8.2 / 7.9;
+// powers of two from L = 1024 as before.
+// A split holds at least 4 tiles, 6 above 8 splits and 8 above 32; and, but
+// for the count of a workgroup per CU, the records fit the scratch array of
+// db_f4_splitkv_noalloc whatever the head group is.
 int f4_choose_splits(int B, int Hkv, int L, int cu_count) {
   const Tuning& t = tuning();
   const int ntiles = (L + kTile - 1) / kTile;
   const int pairs = B * Hkv;
-  const int target = cu_count * t.f4_blocks_per_cu;
-  int S = (target + pairs - 1) / pairs;
-  const int max_by_tiles = ntiles / (t.f4_min_tiles > 0 ? t.f4_min_tiles : 1);
-  S = min(S, max(1, max_by_tiles));
-  S = min(S, 256);
-  return max(S, 1);
+  const int min_tiles = t.f4_min_tiles > 0 ? t.f4_min_tiles : 1;
+  const long target = (long)cu_count * t.f4_blocks_per_cu;
+  long one_round = (target + pairs - 1) / pairs;
+  one_round = min(min(one_round, (long)max(1, ntiles / min_tiles)), 256L);
+  const int S0 = max((int)one_round, 1);
+  const Tuning defaults;
+  if (t.f4_blocks_per_cu != defaults.f4_blocks_per_cu || t.f4_min_tiles != defaults.f4_min_tiles)
+    return S0;
+  if (S0 > 1 && (long)pairs * S0 == cu_count && ntiles % S0 == 0) return S0;  // one full round
+  auto cost = [&](unsigned S) {
+    const unsigned tps = (ntiles + S - 1) / S;
+    const unsigned used = (ntiles + tps - 1) / tps;
+    const unsigned rounds = (unsigned)(((size_t)pairs * used + cu_count - 1) / cu_count);
+    const float merge = used == 1                  ? 0.0f
+                        : used <= kMergeChunk      ? 1.5f
+                        : used <= 16 || used >= 32 ? 2.9f
+                                                   : 3.5f;
+    return 0.3f * (float)rounds * tps + 1.6f * (float)(rounds - 1) + merge;
+  };
+  const size_t per_split = 8 * (sizeof(float2) + kD * sizeof(float));  // 8 heads per pair
+  int best = S0;
+  float least = cost(S0) * 0.95f;  // a change has to be worth 5%
+  auto consider = [&](int S) {
+    if (S < 1 || S > 256 || S > ntiles) return;
+    if (S > 1 && ntiles < S * (S <= kMergeChunk ? 4 : S <= 32 ? 6 : 8)) return;
+    if ((size_t)pairs * (kTicketWords * sizeof(unsigned) + S * per_split) + 512 > kF4ScratchBytes)
+      return;
+    const float c = cost(S);
+    if (c < least) {
+      least = c;
+      best = S;
+    }
+  };
+  // The counts that can win: few splits, the most a tile limit allows, and the
+  // most that 1 to 4 rounds hold.
+  for (int S = 1; S <= kMergeChunk; ++S) consider(S);
+  consider(16);
+  consider(min(32, ntiles / 6));
+  consider(ntiles / 8);
+  for (int k = 1; k <= 4; ++k) consider((int)((long)k * cu_count / pairs));
+  return best;
 }
 
 F4Plan f4_plan(int B, int Hkv, int L, int S, int nxcc, bool allow_fused_merge) {
