@@ -34,12 +34,15 @@
 //    of two (exact) when its first block's mean square is outside [2^-6,
 //    2^14], and streams its columns a second time, scaled by their own mean
 //    square, when a sum is not finite or the first block was not
-//    representative (beyond 2^5 below or 2^8 above).
+//    representative (beyond 2^5 below or 2^8 above).  That second pass takes a
+//    block at a time and the tests fold into one sum: as a second copy of the
+//    pipelined stream with branching tests they cost every call 3-8% (F1 fp16
+//    [7168, 5120] at 24 rows 18.4 us, 17.8 us now; e4m3 [6144, 4096] at 32 12.9, 11.4).
 //
 // Measured on MI355X (graph back to back, us, before / with this kernel): gate/up
 // pair [14336, 4096] at 64 rows fp16 91.0 / 41.1, e4m3 61.9 / 29.4; RMSNorm ->
-// e4m3 gate/up [8201, 3072] at 9 rows 52 / 13.8; F1 [7168, 5120] at 24 rows 115
-// / 18.4; down projection [4096, 11008] at 41 rows 197 / 27.
+// e4m3 gate/up [8201, 3072] at 9 rows 52 / 13.0; F1 [7168, 5120] at 24 rows 115
+// / 17.8; down projection [4096, 11008] at 41 rows 197 / 27.
 #pragma once
 
 #include <type_traits>
@@ -70,16 +73,17 @@ constexpr int tile_lines(bool fp8) { return fp8 ? 2 : 1; }  // x lines per block
 // Waves per workgroup: 8 waves of one tile, 4 of more (2 tiles at 4 rows: 10.5
 // us with 4 waves, 11.3 with 8; 7 tiles at 16 rows 37.3 against 38.7).
 constexpr int tile_waves(int t) { return t == 1 ? 8 : 4; }
-// Blocks in flight per wave: about 26 loads of 1 KB, within the registers that
-// leave the sums and operands unspilled (one block then: F1 e4m3 at 64 rows and
-// one tile 39 us spilled, 17 us).
+// Blocks in flight per wave: about 26 loads of 1 KB, at most 3 (a fourth only
+// adds tail code: e4m3 [6144, 4096] at 4 rows 7.7 us, 7.3 with 3), within the
+// registers that leave the sums and operands unspilled (one block then: F1 e4m3
+// at 64 rows and one tile 39 us spilled, 17 us).
 constexpr int tile_depth(int t, int nxg, bool fp8, bool norm) {
   const int loads = 2 * t + nxg * tile_lines(fp8) + (norm ? tile_lines(fp8) : 0);
   if (t == 1) return 8 * loads + 16 * nxg > 190 ? 1 : 2;
   const int bt = (nxg + 1) / 2;
   const int other = 4 * t * bt + 8 * bt * tile_lines(fp8) + (norm ? 4 * nxg : 0);
   int d = 26 / loads;
-  d = d < 2 ? 2 : d > 4 ? 4 : d;
+  d = d < 2 ? 2 : d > 3 ? 3 : d;
   return 4 * d * loads + other > (norm ? 250 : 290) ? 1 : d;
 }
 
@@ -289,31 +293,35 @@ __global__ __launch_bounds__(tile_waves(T) * kWave) void gemv_tile_kernel(TileAr
     }
     scaled = __any(need);
   };
-  auto stream = [&](bool first) {
+  auto clear = [&]() {
 #pragma unroll
     for (int j = 0; j < T; ++j)
 #pragma unroll
       for (int bt = 0; bt < BT; ++bt) acc[j][bt] = f4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int q = 0; q < NXG; ++q) ss[q] = raw[q] = 0.0f;
+  };
+  auto total_rows = [&]() {
+#pragma unroll
+    for (int q = 0; q < NXG; ++q) ss[q] = row8(scaled ? raw[q] : ss[q]);
+  };
+  auto stream = [&]() {
+    clear();
 #pragma unroll
     for (int d = 0; d < DEPTH; ++d) load_x(d, d);
 #pragma unroll
     for (int d = 0; d < DEPTH; ++d) load_w(d, d);
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (NORM) {
-      if (first) {
-        float sq[NXG];
+      float sq[NXG];
 #pragma unroll
-        for (int q = 0; q < NXG; ++q) {
-          float v = 0.0f;
+      for (int q = 0; q < NXG; ++q) {
+        float v = 0.0f;
 #pragma unroll
-          for (int l = 0; l < LINES; ++l)
-            v = dot8(xs[0][q * LINES + l], xs[0][q * LINES + l], v);
-          sq[q] = row8(v);
-        }
-        set_scale(sq, KB);
+        for (int l = 0; l < LINES; ++l) v = dot8(xs[0][q * LINES + l], xs[0][q * LINES + l], v);
+        sq[q] = row8(v);
       }
+      set_scale(sq, KB);
     }
     int j = 0;
     for (; j + 2 * DEPTH <= n; j += DEPTH) {
@@ -350,38 +358,43 @@ __global__ __launch_bounds__(tile_waves(T) * kWave) void gemv_tile_kernel(TileAr
       case 3: if constexpr (DEPTH >= 2) tail(std::integral_constant<int, 3>{}); break;
       case 4: if constexpr (DEPTH >= 3) tail(std::integral_constant<int, 4>{}); break;
       case 5: if constexpr (DEPTH >= 3) tail(std::integral_constant<int, 5>{}); break;
-      case 6: if constexpr (DEPTH >= 4) tail(std::integral_constant<int, 6>{}); break;
-      case 7: if constexpr (DEPTH >= 4) tail(std::integral_constant<int, 7>{}); break;
       default: break;
     }
-    if constexpr (NORM) {
-#pragma unroll
-      for (int q = 0; q < NXG; ++q) ss[q] = row8(scaled ? raw[q] : ss[q]);
-    }
+    if constexpr (NORM) total_rows();
   };
-  for (bool first = true;; first = false) {
-    stream(first);
-    if constexpr (!NORM) break;
-    if (!first) break;
-    bool bad = false;
+  stream();
+  if constexpr (NORM) {
+    // Straight-line: every test folds into one value that is 0 when all is
+    // well (infinite or NaN sums make 0 x sum NaN).
+    const float per_col = 1.0f / (float)(max(n, 1) * KB);
+    float odd = 0.0f;
 #pragma unroll
     for (int q = 0; q < NXG; ++q) {
       const float f = scaled ? (float)scale[q][0] : 1.0f;
-      const float ms = ss[q] / (float)(n * KB) * f * f;  // NaN without blocks: not bad
-      bad = bad || (ss[q] > 0.0f && (ms < 0x1p-10f || ms > 0x1p16f));
+      const float ms = ss[q] * per_col * f * f;
+      const bool off = (ss[q] > 0.0f) & !((ms >= 0x1p-10f) & (ms <= 0x1p16f));
+      odd += off ? 1.0f : 0.0f;
     }
 #pragma unroll
     for (int j = 0; j < T; ++j)
 #pragma unroll
       for (int bt = 0; bt < BT; ++bt)
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          bad = bad || !(__builtin_fabsf(acc[j][bt][i]) < __builtin_huge_valf());
-    if (!__any(bad)) break;
-    set_scale(ss, n * KB);
-    if (!scaled) break;
-  }
-  if constexpr (NORM) {
+        for (int i = 0; i < 4; ++i) odd = fmaf(acc[j][bt][i], 0.0f, odd);
+    const bool bad = !(odd == 0.0f);
+    if (__builtin_expect(__any(bad), 0)) {
+      set_scale(ss, n * KB);
+      if (scaled) {  // again, a block at a time: rare, and small code
+        clear();
+        for (int j = 0; j < n; ++j) {
+          load_x(0, j);
+          load_w(0, j);
+          stage(0);
+          product();
+        }
+        total_rows();
+      }
+    }
 #pragma unroll
     for (int q = 0; q < NXG; ++q)
       if (lc == 0) {
