@@ -8,6 +8,9 @@ parallel), then linked into ``decodebench_amd/lib/libdecodebench_hip.so``.
 All device code is built with packed-fp32 instructions disabled
 (``-Xclang -target-feature -Xclang -packed-fp32-ops``); the host pass warns
 that it does not know that feature, which is expected.
+
+``csrc/fastcall.cpp``, the native call path of the Python ops, is host code
+built against the installed torch into ``lib/_fastcall.so``.
 """
 
 from __future__ import annotations
@@ -18,6 +21,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
@@ -25,6 +29,8 @@ CSRC = PKG / "csrc"
 BUILD = PKG / "_build"
 LIB_DIR = PKG / "lib"
 LIB = LIB_DIR / "libdecodebench_hip.so"
+FAST_SRC = CSRC / "fastcall.cpp"
+FAST_LIB = LIB_DIR / "_fastcall.so"
 INCLUDE = PKG.parent / "include"
 
 ARCH = os.environ.get("DECODEBENCH_OFFLOAD_ARCH", "gfx950")
@@ -67,16 +73,37 @@ def _compile(src: Path) -> Path:
     return obj
 
 
+def _compile_fast(src: Path) -> Path:
+    import torch
+
+    root = Path(torch.__file__).resolve().parent
+    tmp = FAST_LIB.with_suffix(".so.tmp")
+    abi = int(getattr(torch._C, "_GLIBCXX_USE_CXX11_ABI", True))
+    cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared",
+           f"-D_GLIBCXX_USE_CXX11_ABI={abi}", f"-I{sysconfig.get_paths()['include']}",
+           f"-I{root / 'include'}", f"-I{root / 'include/torch/csrc/api/include'}", str(src),
+           "-o", str(tmp), f"-L{root / 'lib'}", "-ltorch_python", "-ltorch_cpu", "-lc10"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"g++ failed for {src.name}:\n{res.stderr}")
+    os.replace(tmp, FAST_LIB)
+    return FAST_LIB
+
+
 def build(force: bool = False, verbose: bool = True) -> Path:
-    """Compile the HIP library; return the path of the shared object."""
+    """Compile the HIP library and the native call path; return the path of
+    the library."""
     BUILD.mkdir(exist_ok=True)
     LIB_DIR.mkdir(exist_ok=True)
     srcs = _sources()
     todo = [s for s in srcs if force or _stale(BUILD / (s.stem + ".o"), s)]
-    if todo:
-        workers = min(len(todo), max(1, (os.cpu_count() or 2)))
+    jobs = [(_compile, s) for s in todo]
+    if force or _stale(FAST_LIB, FAST_SRC):
+        jobs.insert(0, (_compile_fast, FAST_SRC))
+    if jobs:
+        workers = min(len(jobs), max(1, (os.cpu_count() or 2)))
         with cf.ThreadPoolExecutor(max_workers=workers) as pool:
-            list(pool.map(_compile, todo))
+            list(pool.map(lambda job: job[0](job[1]), jobs))
     objs = [BUILD / (s.stem + ".o") for s in srcs]
     if force or todo or not LIB.exists() or any(
             o.stat().st_mtime > LIB.stat().st_mtime for o in objs):

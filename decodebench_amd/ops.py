@@ -13,6 +13,11 @@ on the current stream) with ctypes over a C ABI instead of a torch extension.
 
 There is no fallback: if the HIP library is missing or cannot be loaded the
 ops raise ``RuntimeError`` naming the build command.
+
+A call that needs nothing but its checks, an output and the launch goes
+through ``_fastcall`` (csrc/fastcall.cpp), which does the same in native code;
+it answers None for everything else, and without it (built for another torch)
+the Python steps below do all of it.
 """
 
 from __future__ import annotations
@@ -23,6 +28,7 @@ import threading
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent / "lib" / "libdecodebench_hip.so"
+FAST_PATH = Path(__file__).resolve().parent / "lib" / "_fastcall.so"
 
 DB_OK = 0
 DB_ERR_INVALID = -1
@@ -32,6 +38,7 @@ DTYPE_FP8_E4M3 = 1
 
 _lock = threading.Lock()
 _lib = None
+_fast = None  # the _fastcall module, once the library is loaded
 _cu_cache: dict[int, int] = {}
 _ws_cache: dict[tuple, object] = {}
 _captured_ws: dict[tuple, object] = {}  # workspaces made under graph capture (kept alive)
@@ -83,8 +90,34 @@ def load_library():
             fn.argtypes = args
         if lib.db_abi_version() != 1:
             raise RuntimeError("libdecodebench_hip.so ABI version mismatch")
+        _load_fast(lib)
         _lib = lib
         return lib
+
+
+def _load_fast(lib) -> None:
+    """Load the native call path and hand it the library's entry points."""
+    global _fast
+    import importlib.machinery
+    import importlib.util
+
+    torch = _torch or _torch_mod()
+    get_device = getattr(torch._C, "_cuda_getDevice", None)
+    if get_device is None or not FAST_PATH.exists():
+        return
+    loader = importlib.machinery.ExtensionFileLoader("_fastcall", str(FAST_PATH))
+    spec = importlib.util.spec_from_file_location("_fastcall", str(FAST_PATH), loader=loader)
+    try:
+        mod = importlib.util.module_from_spec(spec)
+        loader.exec_module(mod)
+    except ImportError:  # built against another torch
+        return
+    entry = tuple(C.cast(getattr(lib, name), C.c_void_p).value for name in (
+        "db_f1_rmsnorm_gemv", "db_f2_gateup_swiglu", "db_f2_rmsnorm_gateup_swiglu", "db_gemv",
+        "db_f4_default_splits", "db_f4_workspace_bytes", "db_f4_splitkv",
+        "db_stream_capture_id"))
+    mod.init(entry, _raw_stream, get_device, _ws_cache, _cu_cache)
+    _fast = mod
 
 
 def _check(rc: int, what: str) -> None:
@@ -271,6 +304,10 @@ def f1_rmsnorm_gemv(x, g, W, eps: float = 1e-6, w_scale=None, out=None):
 
     x [B,K] (or [K]) fp16, g [K] fp16, W [N,K] fp16 (or e4m3 + w_scale [N]).
     Returns [B,N] fp16 (or [N] for a 1-D x), written to ``out`` if given."""
+    if out is None and _fast is not None:
+        y = _fast.f1(x, g, W, eps, w_scale)
+        if y is not None:
+            return y
     torch = _torch or _torch_mod()
     x2, squeeze = _as_2d(x, "x")
     B, K = x2.shape
@@ -291,6 +328,10 @@ def f2_gateup_swiglu(x, Wg, Wu, sg=None, su=None, out=None):
     """F2: ``silu(F.linear(x, Wg)) * F.linear(x, Wu)`` in one kernel.
 
     x [B,K] (or [K]) fp16, Wg/Wu [N,K] fp16 (or e4m3 + per-row scales)."""
+    if out is None and _fast is not None:
+        y = _fast.f2(x, Wg, Wu, sg, su)
+        if y is not None:
+            return y
     torch = _torch or _torch_mod()
     x2, squeeze = _as_2d(x, "x")
     B, K = x2.shape
@@ -314,6 +355,10 @@ def f2_rmsnorm_gateup_swiglu(x, g, Wg, Wu, eps: float = 1e-6, sg=None, su=None, 
 
     x [B,K] (or [K]) fp16, g [K] fp16, Wg/Wu [N,K] fp16 (or e4m3 + per-row
     scales).  Returns [B,N] fp16 (or [N])."""
+    if out is None and _fast is not None:
+        y = _fast.f2n(x, g, Wg, Wu, eps, sg, su)
+        if y is not None:
+            return y
     torch = _torch or _torch_mod()
     x2, squeeze = _as_2d(x, "x")
     B, K = x2.shape
@@ -335,6 +380,10 @@ def f2_rmsnorm_gateup_swiglu(x, g, Wg, Wu, eps: float = 1e-6, sg=None, su=None, 
 
 def gemv(x, W, w_scale=None, out=None):
     """Plain projection ``F.linear(x, W)`` (fp16 out, fp32 accumulation)."""
+    if out is None and _fast is not None:
+        y = _fast.gemv(x, W, w_scale)
+        if y is not None:
+            return y
     torch = _torch or _torch_mod()
     x2, squeeze = _as_2d(x, "x")
     B, K = x2.shape
@@ -415,6 +464,10 @@ def f4_flashdecode(q, K, V, scale: float | None = None, n_splits: int | None = N
     q [B,Hq,D], K/V [B,Hkv,L,D] fp16 (D = 128); query head h reads KV head
     h // (Hq // Hkv).  ``scale`` defaults to 1/sqrt(D); ``n_splits`` defaults
     to the library's CU-count-based choice.  Returns [B,Hq,D] fp16."""
+    if out is None and workspace is None and _fast is not None:
+        o = _fast.f4(q, K, V, scale, n_splits)
+        if o is not None:
+            return o
     torch = _torch or _torch_mod()
     if q.dim() != 3 or K.dim() != 4 or K.shape != V.shape:
         raise ValueError(f"expected q [B,Hq,D] and K, V [B,Hkv,L,D]; got q {tuple(q.shape)}, "
