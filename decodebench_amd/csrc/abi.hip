@@ -145,12 +145,18 @@ dbk::GemvWeights weights(int w_dtype, const void* w0, const void* w1, const floa
 
 int run_gemv(const char* fn, dbk::GemvMode mode, const void* x, const void* g,
              const dbk::GemvWeights& w, void* y, int B, int K, int N, float eps,
-             void* stream) {
+             void* stream, void* ws = nullptr, size_t ws_bytes = 0) {
   int err = 0;
   const int cus = dbk::device_cu_count(&err);
   if (err) return hip_status((hipError_t)err, fn);
-  return hip_status(dbk::launch_gemv(mode, x, g, w, y, B, K, N, eps, cus, (hipStream_t)stream),
+  return hip_status(dbk::launch_gemv(mode, x, g, w, y, B, K, N, eps, cus, ws, ws_bytes,
+                                     (hipStream_t)stream),
                     fn);
+}
+
+dbk::GemvMode gemv_mode(bool norm, bool pair) {
+  return norm ? (pair ? dbk::kGemvRmsNormSwiGLU : dbk::kGemvRmsNorm)
+              : (pair ? dbk::kGemvSwiGLU : dbk::kGemvPlain);
 }
 
 __global__ void null_kernel() {}
@@ -212,6 +218,30 @@ int db_gemv(const void* x, const void* W, const float* w_scale, void* y, int B,
   if (rc) return rc;
   return run_gemv(fn, dbk::kGemvPlain, x, nullptr, weights(w_dtype, W, nullptr, w_scale, nullptr),
                   y, B, K, N, 0.0f, stream);
+}
+
+size_t db_gemv_workspace_bytes(int norm, int pair, int B, int K, int N, int w_dtype) {
+  if (B < 2 || K < 8 || N < 1) return 0;
+  if (w_dtype != DB_DTYPE_F16 && w_dtype != DB_DTYPE_FP8_E4M3) return 0;
+  int err = 0;
+  const int cus = dbk::device_cu_count(&err);
+  if (err) return 0;
+  return dbk::gemv_workspace_bytes(gemv_mode(norm, pair), w_dtype == DB_DTYPE_FP8_E4M3, B, K, N,
+                                   cus);
+}
+
+int db_gemv_ws(const void* x, const void* g, const void* W, const void* W2, const float* scale,
+               const float* scale2, void* y, void* ws, size_t ws_bytes, int B, int K, int N,
+               float eps, int w_dtype, void* stream) {
+  const char* fn = "db_gemv_ws";
+  int rc = g ? check_norm(fn, g, eps) : DB_OK;
+  if (!rc) rc = check_gemv(fn, x, W, y, B, K, N, w_dtype, scale, W2, scale2, W2 != nullptr);
+  if (rc) return rc;
+  if (ws && !aligned16(ws))
+    return fail(DB_ERR_INVALID, "%s: workspace must be 16-byte aligned", fn);
+  return run_gemv(fn, gemv_mode(g != nullptr, W2 != nullptr), x, g,
+                  weights(w_dtype, W, W2, scale, scale2), y, B, K, N, g ? eps : 0.0f, stream, ws,
+                  ws ? ws_bytes : 0);
 }
 
 int db_f4_default_splits(int B, int Hkv, int L, int cu_count) {
@@ -305,6 +335,8 @@ const Knob kKnobs[] = {
      nullptr},
     {"gemv_tile", &dbk::Tuning::gemv_tile, [](int v) { return v >= 0 && v <= 2; },
      "0 (automatic), 1 or 2", nullptr},
+    {"gemv_splits", &dbk::Tuning::gemv_splits, [](int v) { return v >= 0 && v <= 8; },
+     "0 (automatic) to 8", nullptr},
     {"f4_launch", &dbk::Tuning::f4_launch, [](int v) { return v >= 0 && v <= 2; },
      "0 (both launches), 1 (split kernel only) or 2 (merge only)", nullptr},
 };

@@ -38,6 +38,7 @@ struct Tuning {
                                // full grid instead
   int gemv_tile = 0;           // batches of 2 rows and more (gemv_mfma_min_batch if set):
                                // 0 automatic, 1 gemv_tile, 2 never gemv_tile
+  int gemv_splits = 0;         // K splits of gemv_tile where a workspace is given: 0 auto, 1..8
   int f4_launch = 0;           // measurement hook for the two-launch F4: 0 both
                                // launches, 1 the split kernel only, 2 the merge only
 };
@@ -79,9 +80,13 @@ struct GemvWeights {
 //   kGemvRmsNormSwiGLU  : the SwiGLU mode on the RMS-normalised x
 // With fp8 weights every projection is fp32(sum) * row scale before its
 // fp16 rounding.
+// ws (ws_bytes of device memory, 16-byte aligned, or null) lets a call that
+// gains from it split K over workgroups, see gemv_workspace_bytes.
 hipError_t launch_gemv(GemvMode mode, const void* x, const void* gamma,
                        const GemvWeights& w, void* y, int B, int K, int N, float eps,
-                       int cu_count, hipStream_t stream);
+                       int cu_count, void* ws, size_t ws_bytes, hipStream_t stream);
+// Bytes of workspace with which launch_gemv would split K (0: it would not).
+size_t gemv_workspace_bytes(GemvMode mode, bool fp8, int B, int K, int N, int cu_count);
 
 // MFMA variant for batches of up to 16 rows per pass (gemv_mfma.hip), fp16
 // or e4m3 weights, K in {2048, 4096}.
@@ -92,9 +97,11 @@ hipError_t launch_gemv_mfma(GemvMode mode, const void* x, const void* gamma,
 
 // Batched GEMV on full 16 x 16 MFMA tiles with streamed activations
 // (gemv_tile.hip): any K the contract allows, any N and batch.
+// With splits > 1 the partial sums go to ws and a second launch adds them.
+size_t gemv_tile_workspace_bytes(GemvMode mode, int splits, int B, int N);
 hipError_t launch_gemv_tile(GemvMode mode, const void* x, const void* gamma,
                             const GemvWeights& w, void* y, int B, int K, int N, float eps,
-                            int cu_count, hipStream_t stream);
+                            int cu_count, int splits, void* ws, hipStream_t stream);
 
 // Split-KV GQA decode attention with the log-sum-exp combine in-kernel.
 size_t f4_workspace_bytes(int B, int Hq, int Hkv, int S, int D);

@@ -34,6 +34,8 @@ struct Abi {
   decltype(&db_f4_workspace_bytes) f4_workspace_bytes;
   decltype(&db_f4_splitkv) f4;
   decltype(&db_stream_capture_id) capture_id;
+  decltype(&db_gemv_workspace_bytes) gemv_workspace_bytes;
+  decltype(&db_gemv_ws) gemv_ws;
 } abi;
 
 PyObject* raw_stream = nullptr;  // device index -> current stream's handle
@@ -135,9 +137,18 @@ PyObject* gemv_op(PyObject* xo, PyObject* go, PyObject* w0o, PyObject* w1o, PyOb
   const void* w1p = w1 ? w1->data_ptr() : nullptr;
   void* yp = y.data_ptr();
   const int b = (int)B, k = (int)K, n = (int)N;
+  // K split over workgroups, in a workspace that the allocator takes back in
+  // stream order after this call.
+  at::Tensor ws;
+  const size_t bytes = b > 8 ? abi.gemv_workspace_bytes(g != nullptr, w1 != nullptr, b, k, n, dtype) : 0;
+  if (bytes > 0)
+    ws = at::empty({(int64_t)bytes}, at::TensorOptions().dtype(at::kByte).device(y.device()));
+  void* wsp = bytes > 0 ? ws.data_ptr() : nullptr;
   int rc;
   Py_BEGIN_ALLOW_THREADS
-  if (w1)
+  if (bytes > 0)
+    rc = abi.gemv_ws(xp, gp, w0p, w1p, s0, s1, yp, wsp, bytes, b, k, n, (float)eps, dtype, stream);
+  else if (w1)
     rc = g ? abi.f2n(xp, gp, w0p, w1p, s0, s1, yp, b, k, n, (float)eps, dtype, stream)
            : abi.f2(xp, w0p, w1p, s0, s1, yp, b, k, n, dtype, stream);
   else
@@ -255,10 +266,10 @@ PyObject* f4(PyObject*, PyObject* const* a, Py_ssize_t n) {
 
 // (entry point addresses, raw_stream, get_device, workspaces, cu_counts)
 PyObject* init(PyObject*, PyObject* args) {
-  unsigned long long p[8];
+  unsigned long long p[10];
   PyObject *rs, *gd, *ws, *cu;
-  if (!PyArg_ParseTuple(args, "(KKKKKKKK)OOO!O!", &p[0], &p[1], &p[2], &p[3], &p[4], &p[5], &p[6],
-                        &p[7], &rs, &gd, &PyDict_Type, &ws, &PyDict_Type, &cu))
+  if (!PyArg_ParseTuple(args, "(KKKKKKKKKK)OOO!O!", &p[0], &p[1], &p[2], &p[3], &p[4], &p[5], &p[6],
+                        &p[7], &p[8], &p[9], &rs, &gd, &PyDict_Type, &ws, &PyDict_Type, &cu))
     return nullptr;
   abi.f1 = reinterpret_cast<decltype(abi.f1)>((uintptr_t)p[0]);
   abi.f2 = reinterpret_cast<decltype(abi.f2)>((uintptr_t)p[1]);
@@ -268,6 +279,8 @@ PyObject* init(PyObject*, PyObject* args) {
   abi.f4_workspace_bytes = reinterpret_cast<decltype(abi.f4_workspace_bytes)>((uintptr_t)p[5]);
   abi.f4 = reinterpret_cast<decltype(abi.f4)>((uintptr_t)p[6]);
   abi.capture_id = reinterpret_cast<decltype(abi.capture_id)>((uintptr_t)p[7]);
+  abi.gemv_workspace_bytes = reinterpret_cast<decltype(abi.gemv_workspace_bytes)>((uintptr_t)p[8]);
+  abi.gemv_ws = reinterpret_cast<decltype(abi.gemv_ws)>((uintptr_t)p[9]);
   Py_INCREF(rs);
   Py_INCREF(gd);
   Py_INCREF(ws);

@@ -10,7 +10,7 @@
 #include <mutex>
 #include <unordered_map>
 
-#include "gemv_valu.h"
+#include "gemv_tile.h"
 
 namespace dbk {
 
@@ -80,7 +80,10 @@ GemvFn gemv_pick_f1_two_rows(int u) {
 //  * The plain projection: 3 rows and more (fp16 [4096, 4096] at 8, 24 and
 //    64 rows 8.9 / 8.6, 12.8 / 10.8, 19.8 / 14.6); at K = 2048 only with
 //    more than a tile per CU ([2048, 2048] at 16 rows 5.0 / 5.2); e4m3 with one
-//    tile per CU to 12 rows (6.8 / 6.2 at 8, 7.3 / 7.5 at 16).
+//    tile per CU to 12 rows (6.8 / 6.2 at 8, 7.3 / 7.5 at 16).  To 3072
+//    outputs (12 per CU) 16-row passes side by side read less of x ([1024,
+//    4096] at 4 and 32 rows 5.6 / 6.1, 6.1 / 7.1; F1 6.4 / 8.9 at 24), but for
+//    2048 and more above 32 rows.
 //  * Its rows longer than 4096, above 8 outputs per CU: [4096, 14336] fp16
 //    at 16 rows 28.0 / 25.2, e4m3 at 8 rows 16.0 / 14.8; [1024, 8192] 7.3 /
 //    8.4 stays, and so do one-tile e4m3 calls above 48 rows (33.9 / 35.6).
@@ -100,13 +103,59 @@ bool tile_gemv(GemvMode mode, bool fp8, int B, int K, int N) {
     return !forced && N > 2048 && !(fp8 && one_tile && B > 48);
   }
   if (t.gemv_xb != 0 || t.gemv_pass_grid != 0) return false;
+  if (N <= 3072) return !fp8 && K == 4096 && N >= 2048 && B > 32;
   if (mode == kGemvRmsNorm)
     return !fp8 && K == 4096 && B >= 17 && (!one_tile || B <= 24 || B > 32);
   if (K < 4096) return !one_tile && B >= 3;
   return fp8 ? (B >= 3 && B <= 12) || (B >= 17 && !one_tile) : B >= 3;
 }
 
+// K splits of a call that has a workspace, 1 where one launch is as fast.
+// Each CU reads all of x for its rows, so with many rows or long ones x, not
+// its share of the weights, fills its L1: 14336 columns of 64 rows are 1.8 MB
+// beside 0.45 MB of fp16 weights at N = 4096.  S workgroups with S times the
+// outputs and 1 / S of the columns read x / S each.  They pay for it with S
+// partial sums per output and a second launch, about 1.5 us and 0.7 us per
+// tile (1.4 for the pair) against the 52 GB/s at which a CU reads x between
+// weights.  Measured on MI355X (us, one launch / 4 splits): fp16 [4096, 14336] at
+// 12, 24 and 64 rows 23.2 / 23.1, 30.3 / 24.2, 44.3 / 28.8, e4m3 at 64 34.1 /
+// 23.7; [4096, 11008] at 12 and 41 rows 18.7 / 19.0, 27.8 / 21.6; [1024, 4096]
+// at 64 11.5 / 8.3; [4096, 4096] at 24 and 64 10.5 / 11.2, 14.7 / 13.3; pair
+// [2048, 8192] at 24 and 64 17.3 / 17.9, 24.9 / 21.4.  2 and 8 splits were
+// behind 4, and 3 ahead where they fill the CUs with 4 tiles and 4 splits take
+// 5 ([5120, 5120] at 41 rows 19.8 / 16.4 / 17.0); more than 4 tiles gained
+// nothing (e4m3 F1 [7168, 5120] at 64 rows 20.7 / 22.8), nor did short rows
+// ([2048, 2048] at 64 7.3 / 8.5).
+int tile_splits(GemvMode mode, bool fp8, int B, int K, int N, int cu_count) {
+  const bool pair = gemv_is_swiglu(mode);
+  const int forced = tuning().gemv_splits;
+  // Tiles per workgroup with S splits, 0 where there are too few columns.
+  auto tiles = [&](int S) {
+    const int slots = cu_count / S / 8 * 8;
+    const int blocks = (K + (fp8 ? 127 : 63)) / (fp8 ? 128 : 64);
+    const int t = slots < 8 || blocks < 4 * S
+                      ? 0
+                      : ((N + slots - 1) / slots + (pair ? 7 : 15)) / (pair ? 8 : 16);
+    return t <= kTileMaxTiles ? t : 0;
+  };
+  if (forced > 0) return tiles(forced) > 0 ? forced : 1;
+  const float x_kb = (float)B * (float)K * (2.0f / 1024.0f);
+  if (B < 9 || K < 3072 || x_kb < 250.0f) return 1;
+  if (K <= 4096 && !tile_gemv(mode, fp8, B, K, N)) return 1;
+  const int S = tiles(4) > 4 && tiles(3) > 0 && tiles(3) <= 4 ? 3 : 4;
+  const int t = tiles(S);
+  if (t == 0 || t > 4) return 1;
+  const float gain = x_kb * (1.0f - 1.0f / (float)S) / 52.0f;
+  return gain > 2.0f + (pair ? 1.4f : 0.7f) * (float)t ? S : 1;
+}
+
 }  // namespace
+
+size_t gemv_workspace_bytes(GemvMode mode, bool fp8, int B, int K, int N, int cu_count) {
+  const int forced_min = tuning().gemv_mfma_min_batch;
+  if (B < (forced_min > 0 ? forced_min : 2)) return 0;
+  return gemv_tile_workspace_bytes(mode, tile_splits(mode, fp8, B, K, N, cu_count), B, N);
+}
 
 hipError_t allow_large_lds(const void* fn, size_t dynamic_bytes) {
   static std::mutex mu;
@@ -130,7 +179,7 @@ hipError_t allow_large_lds(const void* fn, size_t dynamic_bytes) {
 
 hipError_t launch_gemv(GemvMode mode, const void* x, const void* gamma,
                        const GemvWeights& w, void* y, int B, int K, int N, float eps,
-                       int cu_count, hipStream_t stream) {
+                       int cu_count, void* ws, size_t ws_bytes, hipStream_t stream) {
   const int forced_min = tuning().gemv_mfma_min_batch;
   // Where gemv_mfma.hip takes the width.  At 3 rows the VALU kernel would run two 2-row passes, 1.5-1.8x the MFMA
   // time.  At 2 rows (graph back-to-back, us, VALU / MFMA) MFMA takes the
@@ -144,8 +193,12 @@ hipError_t launch_gemv(GemvMode mode, const void* x, const void* gamma,
   const bool mfma_at_two = (w.fp8 && mode != kGemvPlain) || (mode == kGemvPlain && K > 4096);
   const int auto_min = mfma_at_two ? 2 : 3;
   const int mfma_min = forced_min > 0 ? forced_min : auto_min;
-  if (B >= (forced_min > 0 ? forced_min : 2) && tile_gemv(mode, w.fp8, B, K, N))
-    return launch_gemv_tile(mode, x, gamma, w, y, B, K, N, eps, cu_count, stream);
+  if (B >= (forced_min > 0 ? forced_min : 2)) {
+    int splits = ws ? tile_splits(mode, w.fp8, B, K, N, cu_count) : 1;
+    if (gemv_tile_workspace_bytes(mode, splits, B, N) > ws_bytes) splits = 1;
+    if (splits > 1 || tile_gemv(mode, w.fp8, B, K, N))
+      return launch_gemv_tile(mode, x, gamma, w, y, B, K, N, eps, cu_count, splits, ws, stream);
+  }
   if (B >= mfma_min && gemv_mfma_supported(mode, B, K, N))
     return launch_gemv_mfma(mode, x, gamma, w, y, B, K, N, eps, cu_count, stream);
   GemvArgs a;

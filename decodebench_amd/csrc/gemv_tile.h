@@ -62,6 +62,10 @@ struct TileArgs {
   int B, K, N;
   int rows;               // outputs per workgroup (a multiple of 4)
   float eps;
+  int splits;             // K splits (grid.z)
+  f4* part;               // splits > 1: [splits][1 or 2 matrices][ceil(N / 4)][B] partial
+                          // sums of 4 outputs
+  float* ssq;             // splits > 1, norm modes: [splits][B] sums of x^2
 };
 using TileFn = void (*)(TileArgs);
 
@@ -95,6 +99,44 @@ TileFn gemv_tile_pick_fp8(bool norm, int t, int nxg);
 TileFn gemv_tile_pick_fp8_pair(bool norm, int t, int nxg);
 
 namespace {
+
+// Outputs row .. row + 3 (below end) of batch row n from their fp32 sums.
+template <bool FP8, bool NORM, bool PAIR>
+__device__ __forceinline__ void tile_outputs(const TileArgs& a, const f4& s0, const f4& s1,
+                                             float sum_sq, int n, int row, int end) {
+  const float inv = NORM ? 1.0f / sqrtf(sum_sq / (float)a.K + a.eps) : 1.0f;
+  _Float16* const yp = a.y + (size_t)n * a.N + row;
+  _Float16 out[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = min(row + i, a.N - 1);
+    float p = s0[i], u = s1[i];
+    if constexpr (NORM) {
+      p *= inv;
+      u *= inv;
+    }
+    if constexpr (FP8) {
+      p *= a.s0[r];
+      if constexpr (PAIR) u *= a.s1[r];
+    }
+    if constexpr (PAIR) {
+      const float gq = (float)to_h(p);
+      const float uq = (float)to_h(u);
+      p = (float)to_h(gemv_silu(gq)) * uq;
+    }
+    out[i] = to_h(p);
+  }
+  if ((a.N & 3) == 0) {  // then row and N are multiples of 4: one aligned store
+    uint2 v;
+    v.x = __builtin_bit_cast(unsigned, h2{out[0], out[1]});
+    v.y = __builtin_bit_cast(unsigned, h2{out[2], out[3]});
+    *reinterpret_cast<uint2*>(yp) = v;
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (row + i < end) yp[i] = out[i];
+  }
+}
 
 template <int T, int NXG, bool FP8, bool NORM, bool PAIR>
 __global__ __launch_bounds__(tile_waves(T) * kWave) void gemv_tile_kernel(TileArgs a) {
@@ -160,15 +202,18 @@ __global__ __launch_bounds__(tile_waves(T) * kWave) void gemv_tile_kernel(TileAr
   const __amdgpu_buffer_rsrc_t rx = make_rsrc(a.x + (size_t)b0 * a.K, kRange);
   const __amdgpu_buffer_rsrc_t rg = make_rsrc(NORM ? a.gamma : a.x, kRange);
 
-  // k-blocks, dealt to the waves in turn; each workgroup starts at a position
+  // The split's k-blocks, dealt to the waves in turn; each workgroup starts at a position
   // of its own, so that the workgroups read x out of step.
   const int nkb = (a.K + KB - 1) / KB;
-  const int n = wave < nkb ? (nkb - wave + WV - 1) / WV : 0;
+  const int split = blockIdx.z;
+  const int kb0 = (int)((unsigned)nkb * split / (unsigned)a.splits);
+  const int nks = (int)((unsigned)nkb * (split + 1) / (unsigned)a.splits) - kb0;
+  const int n = wave < nks ? (nks - wave + WV - 1) / WV : 0;
   const int rot = n > 0 ? (bx + (bx >> 3)) % n : 0;
   auto block_col = [&](int j) {
     int i = j + rot;
     i = i >= n ? i - n : i;
-    return j < n ? (wave + WV * i) * KB : a.K;
+    return j < n ? (kb0 + wave + WV * i) * KB : a.K;
   };
 
   u4 ws[DEPTH][NG];
@@ -439,43 +484,22 @@ __global__ __launch_bounds__(tile_waves(T) * kWave) void gemv_tile_kernel(TileAr
       s0 += part[(v * T * BT + jb) * kWave + l];
       if constexpr (PAIR) s1 += part[(v * T * BT + jb) * kWave + l + 32];
     }
-    float inv = 1.0f;
+    float tot = 0.0f;
     if constexpr (NORM) {
-      float tot = 0.0f;
 #pragma unroll
       for (int v = 0; v < WV; ++v) tot += red[v][nn];
-      inv = 1.0f / sqrtf(tot / (float)a.K + a.eps);
     }
-    _Float16* const yp = a.y + (size_t)(b0 + nn) * a.N + r0 + ob;
-    _Float16 out[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int row = min(r0 + ob + i, a.N - 1);
-      float p = s0[i], u = s1[i];
+    if (a.splits > 1) {
+      const size_t n4 = (a.N + 3) / 4;
+      f4* const pp =
+          a.part + ((size_t)split * (PAIR ? 2 : 1) * n4 + (r0 + ob) / 4) * a.B + b0 + nn;
+      pp[0] = s0;
+      if constexpr (PAIR) pp[n4 * a.B] = s1;
       if constexpr (NORM) {
-        p *= inv;
-        u *= inv;
+        if (bx == 0 && ob == 0) a.ssq[(size_t)split * a.B + b0 + nn] = tot;
       }
-      if constexpr (FP8) {
-        p *= a.s0[row];
-        if constexpr (PAIR) u *= a.s1[row];
-      }
-      if constexpr (PAIR) {
-        const float gq = (float)to_h(p);
-        const float uq = (float)to_h(u);
-        p = (float)to_h(gemv_silu(gq)) * uq;
-      }
-      out[i] = to_h(p);
-    }
-    if ((a.N & 3) == 0) {  // then r0 + ob and N are multiples of 4: one aligned store
-      uint2 v;
-      v.x = __builtin_bit_cast(unsigned, h2{out[0], out[1]});
-      v.y = __builtin_bit_cast(unsigned, h2{out[2], out[3]});
-      *reinterpret_cast<uint2*>(yp) = v;
     } else {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (ob + i < nr) yp[i] = out[i];
+      tile_outputs<FP8, NORM, PAIR>(a, s0, s1, tot, b0 + nn, r0 + ob, r0 + nr);
     }
   }
 }

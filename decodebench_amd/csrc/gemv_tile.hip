@@ -3,9 +3,54 @@
 
 namespace dbk {
 
+namespace {
+
+// Second launch of a call with K splits: thread (n, r4) adds the splits of
+// outputs 4 r4 .. + 3 of batch row n.  A workgroup covers 16 batch rows x 16
+// quads, one 128-byte line of y per batch row, and reads 256 contiguous bytes
+// per quad and split.
+template <bool FP8, bool NORM, bool PAIR>
+__global__ __launch_bounds__(256) void gemv_tile_combine(TileArgs a) {
+  const int n = blockIdx.y * 16 + (threadIdx.x & 15);
+  const int r4 = blockIdx.x * 16 + (threadIdx.x >> 4);
+  const int n4 = (a.N + 3) / 4;
+  if (n >= a.B || r4 >= n4) return;
+  constexpr int NWM = PAIR ? 2 : 1;
+  const size_t stride = (size_t)n4 * a.B;
+  const f4* const pp = a.part + (size_t)r4 * a.B + n;
+  f4 s0 = {0.0f, 0.0f, 0.0f, 0.0f}, s1 = s0;
+  float tot = 0.0f;
+#pragma unroll 4
+  for (int s = 0; s < a.splits; ++s) {
+    s0 += pp[stride * NWM * s];
+    if constexpr (PAIR) s1 += pp[stride * (NWM * s + 1)];
+    if constexpr (NORM) tot += a.ssq[(size_t)s * a.B + n];
+  }
+  tile_outputs<FP8, NORM, PAIR>(a, s0, s1, tot, n, 4 * r4, a.N);
+}
+
+template <bool FP8>
+TileFn combine_pick(bool norm, bool pair) {
+  if (norm) return pair ? gemv_tile_combine<FP8, true, true> : gemv_tile_combine<FP8, true, false>;
+  return pair ? gemv_tile_combine<FP8, false, true> : gemv_tile_combine<FP8, false, false>;
+}
+
+size_t part_bytes(int splits, bool pair, int B, int N) {
+  return (size_t)splits * (pair ? 2 : 1) * ((N + 3) / 4) * B * sizeof(f4);
+}
+
+}  // namespace
+
+// Workspace: the partial sums, then (norm modes) the sums of x^2.
+size_t gemv_tile_workspace_bytes(GemvMode mode, int splits, int B, int N) {
+  return splits <= 1 ? 0
+                     : part_bytes(splits, gemv_is_swiglu(mode), B, N) +
+                           (size_t)splits * B * sizeof(float);
+}
+
 hipError_t launch_gemv_tile(GemvMode mode, const void* x, const void* gamma, const GemvWeights& w,
-                            void* y, int B, int K, int N, float eps, int cu_count,
-                            hipStream_t stream) {
+                            void* y, int B, int K, int N, float eps, int cu_count, int splits,
+                            void* ws, hipStream_t stream) {
   const bool norm = gemv_has_norm(mode), pair = gemv_is_swiglu(mode);
   TileArgs a;
   a.x = static_cast<const _Float16*>(x);
@@ -19,6 +64,10 @@ hipError_t launch_gemv_tile(GemvMode mode, const void* x, const void* gamma, con
   a.K = K;
   a.N = N;
   a.eps = eps;
+  a.splits = splits;
+  a.part = static_cast<f4*>(ws);
+  a.ssq = ws ? reinterpret_cast<float*>(static_cast<char*>(ws) + part_bytes(splits, pair, B, N))
+             : nullptr;
   // Batch rows per pass: the fewest groups of 8 that hold an even share.
   const int passes = (B + 8 * kTileMaxGroups - 1) / (8 * kTileMaxGroups);
   int nxg = ((B + passes - 1) / passes + 7) / 8;
@@ -26,7 +75,7 @@ hipError_t launch_gemv_tile(GemvMode mode, const void* x, const void* gamma, con
   // Outputs per workgroup: an even share of a workgroup per CU (of several
   // rounds of them where a share would be more than 8 tiles).
   const int per = pair ? 8 : 16;
-  const int slots = max(8, cu_count / passes / 8 * 8);
+  const int slots = max(8, cu_count / passes / splits / 8 * 8);
   const int rounds = (N + slots * per * kTileMaxTiles - 1) / (slots * per * kTileMaxTiles);
   a.rows = ((N + slots * rounds - 1) / (slots * rounds) + 3) / 4 * 4;
   const int t = (a.rows + per - 1) / per;
@@ -42,8 +91,14 @@ hipError_t launch_gemv_tile(GemvMode mode, const void* x, const void* gamma, con
     hipError_t e = allow_large_lds(reinterpret_cast<const void*>(fn), lds);
     if (e != hipSuccess) return e;
   }
-  dim3 g(grid, (B + 8 * nxg - 1) / (8 * nxg));
+  dim3 g(grid, (B + 8 * nxg - 1) / (8 * nxg), splits);
   hipLaunchKernelGGL(fn, g, dim3(wv * kWave), lds, stream, a);
+  if (splits > 1) {
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    const TileFn add = w.fp8 ? combine_pick<true>(norm, pair) : combine_pick<false>(norm, pair);
+    hipLaunchKernelGGL(add, dim3(((N + 3) / 4 + 15) / 16, (B + 15) / 16), dim3(256), 0, stream, a);
+  }
   return hipGetLastError();
 }
 

@@ -1,7 +1,8 @@
 """Fused decode ops backed by libdecodebench_hip.so (HIP, gfx950).
 
 Each op takes torch tensors on the GPU, allocates its output with
-``torch.empty`` and launches one kernel on ``torch.cuda.current_stream()``
+``torch.empty`` and launches one kernel (two where K is split over workgroups
+or an F4 merge takes a launch of its own) on ``torch.cuda.current_stream()``
 through the C ABI declared in ``include/decodebench_hip.h``.  No op allocates
 inside the library, synchronises, or reads device memory on the host, so the
 ops work as ``Sequence`` stages, inside a ``profile(fused=...)`` callable, and
@@ -71,6 +72,9 @@ def load_library():
             "db_f2_rmsnorm_gateup_swiglu": (_i, [_p, _p, _p, _p, _p, _p, _p, _i, _i, _i,
                                                  C.c_float, _i, _p]),
             "db_gemv": (_i, [_p, _p, _p, _p, _i, _i, _i, _i, _p]),
+            "db_gemv_workspace_bytes": (C.c_size_t, [_i, _i, _i, _i, _i, _i]),
+            "db_gemv_ws": (_i, [_p, _p, _p, _p, _p, _p, _p, _p, C.c_size_t, _i, _i, _i, C.c_float,
+                                _i, _p]),
             "db_f4_default_splits": (_i, [_i, _i, _i, _i]),
             "db_f4_workspace_bytes": (C.c_size_t, [_i, _i, _i, _i, _i, _i]),
             "db_f4_splitkv": (_i, [_p, _p, _p, _p, _p, C.c_size_t, _i, _i, _i, _i, _i, _i,
@@ -115,7 +119,7 @@ def _load_fast(lib) -> None:
     entry = tuple(C.cast(getattr(lib, name), C.c_void_p).value for name in (
         "db_f1_rmsnorm_gemv", "db_f2_gateup_swiglu", "db_f2_rmsnorm_gateup_swiglu", "db_gemv",
         "db_f4_default_splits", "db_f4_workspace_bytes", "db_f4_splitkv",
-        "db_stream_capture_id"))
+        "db_stream_capture_id", "db_gemv_workspace_bytes", "db_gemv_ws"))
     mod.init(entry, _raw_stream, get_device, _ws_cache, _cu_cache)
     _fast = mod
 
@@ -299,6 +303,23 @@ def _as_2d(x, name: str):
     return x, False
 
 
+def _split_launch(out, x, g, W, W2, s, s2, y, B: int, K: int, N: int, eps: float, dt: int,
+                  idx: int) -> bool:
+    """Launch a GEMV op with K split over workgroups, in a workspace from
+    torch's allocator, where the library would (``db_gemv_workspace_bytes``).
+    Returns whether it did; a call with its own ``out`` allocates nothing, and
+    a refused one is left to the entry point without a workspace."""
+    torch, lib = _torch, _lib or load_library()
+    if out is not None or B < 9 or torch.cuda.current_device() != idx:
+        return False
+    nbytes = lib.db_gemv_workspace_bytes(g is not None, W2 is not None, B, K, N, dt)
+    if nbytes == 0:
+        return False
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=y.device)
+    return lib.db_gemv_ws(x, g, W, W2, s, s2, y.data_ptr(), ws.data_ptr(), nbytes, B, K, N, eps,
+                          dt, _raw_stream(idx)) == DB_OK
+
+
 def f1_rmsnorm_gemv(x, g, W, eps: float = 1e-6, w_scale=None, out=None):
     """F1: ``F.linear(rmsnorm(x, g, eps), W)`` in one kernel.
 
@@ -318,9 +339,11 @@ def f1_rmsnorm_gemv(x, g, W, eps: float = 1e-6, w_scale=None, out=None):
     dt, sp, sc = _weights(W, w_scale, "W", N, K)
     idx = _gpu_tensors((x, "x", torch.float16), (g, "g", torch.float16), (W, "W", None), *sc)
     y = _output((B, N), idx, out)
-    _launch((_lib or load_library()).db_f1_rmsnorm_gemv, idx, "db_f1_rmsnorm_gemv",
-            x2.data_ptr(), g.data_ptr(), W.data_ptr(), sp, y.data_ptr(), B, K, N,
-            float(eps), dt)
+    if not _split_launch(out, x2.data_ptr(), g.data_ptr(), W.data_ptr(), None, sp, None, y, B, K,
+                         N, float(eps), dt, idx):
+        _launch((_lib or load_library()).db_f1_rmsnorm_gemv, idx, "db_f1_rmsnorm_gemv",
+                x2.data_ptr(), g.data_ptr(), W.data_ptr(), sp, y.data_ptr(), B, K, N,
+                float(eps), dt)
     return y[0] if squeeze else y
 
 
@@ -343,8 +366,10 @@ def f2_gateup_swiglu(x, Wg, Wu, sg=None, su=None, out=None):
     _, sup, suc = _weights(Wu, su, "Wu", N, K)
     idx = _gpu_tensors((x, "x", torch.float16), (Wg, "Wg", None), (Wu, "Wu", None), *sgc, *suc)
     y = _output((B, N), idx, out)
-    _launch((_lib or load_library()).db_f2_gateup_swiglu, idx, "db_f2_gateup_swiglu",
-            x2.data_ptr(), Wg.data_ptr(), Wu.data_ptr(), sgp, sup, y.data_ptr(), B, K, N, dt)
+    if not _split_launch(out, x2.data_ptr(), None, Wg.data_ptr(), Wu.data_ptr(), sgp, sup, y, B,
+                         K, N, 0.0, dt, idx):
+        _launch((_lib or load_library()).db_f2_gateup_swiglu, idx, "db_f2_gateup_swiglu",
+                x2.data_ptr(), Wg.data_ptr(), Wu.data_ptr(), sgp, sup, y.data_ptr(), B, K, N, dt)
     return y[0] if squeeze else y
 
 
@@ -372,9 +397,11 @@ def f2_rmsnorm_gateup_swiglu(x, g, Wg, Wu, eps: float = 1e-6, sg=None, su=None, 
     idx = _gpu_tensors((x, "x", torch.float16), (g, "g", torch.float16), (Wg, "Wg", None),
                        (Wu, "Wu", None), *sgc, *suc)
     y = _output((B, N), idx, out)
-    _launch((_lib or load_library()).db_f2_rmsnorm_gateup_swiglu, idx,
-            "db_f2_rmsnorm_gateup_swiglu", x2.data_ptr(), g.data_ptr(), Wg.data_ptr(),
-            Wu.data_ptr(), sgp, sup, y.data_ptr(), B, K, N, float(eps), dt)
+    if not _split_launch(out, x2.data_ptr(), g.data_ptr(), Wg.data_ptr(), Wu.data_ptr(), sgp, sup,
+                         y, B, K, N, float(eps), dt, idx):
+        _launch((_lib or load_library()).db_f2_rmsnorm_gateup_swiglu, idx,
+                "db_f2_rmsnorm_gateup_swiglu", x2.data_ptr(), g.data_ptr(), Wg.data_ptr(),
+                Wu.data_ptr(), sgp, sup, y.data_ptr(), B, K, N, float(eps), dt)
     return y[0] if squeeze else y
 
 
@@ -393,8 +420,10 @@ def gemv(x, W, w_scale=None, out=None):
     dt, sp, sc = _weights(W, w_scale, "W", N, K)
     idx = _gpu_tensors((x, "x", torch.float16), (W, "W", None), *sc)
     y = _output((B, N), idx, out)
-    _launch((_lib or load_library()).db_gemv, idx, "db_gemv",
-            x2.data_ptr(), W.data_ptr(), sp, y.data_ptr(), B, K, N, dt)
+    if not _split_launch(out, x2.data_ptr(), None, W.data_ptr(), None, sp, None, y, B, K, N, 0.0,
+                         dt, idx):
+        _launch((_lib or load_library()).db_gemv, idx, "db_gemv",
+                x2.data_ptr(), W.data_ptr(), sp, y.data_ptr(), B, K, N, dt)
     return y[0] if squeeze else y
 
 

@@ -106,9 +106,29 @@ int db_f2_rmsnorm_gateup_swiglu(const void* x, const void* g, const void* Wg,
 int db_gemv(const void* x, const void* W, const float* w_scale, void* y,
             int B, int K, int N, int w_dtype, void* stream);
 
+/* Bytes of caller-owned workspace with which db_gemv_ws would split the K
+ * columns of such a call over workgroups on the current device (norm, pair:
+ * 1 with a gain, with two matrices); 0 where one launch is as fast, for
+ * arguments the entry points refuse, or without a device.  No counterpart in
+ * the reference. */
+size_t db_gemv_workspace_bytes(int norm, int pair, int B, int K, int N, int w_dtype);
+
+/* db_gemv (g and W2 NULL), db_f1_rmsnorm_gemv (g), db_f2_gateup_swiglu (W2) or
+ * db_f2_rmsnorm_gateup_swiglu (both) with a workspace.  Where
+ * db_gemv_workspace_bytes is not 0 and ws holds that many bytes, workgroups
+ * sum parts of K into it and a second launch on the same stream adds the parts
+ * and writes y; otherwise (ws NULL or too small) the call is the one without a
+ * workspace.  The workspace needs no initialisation and holds nothing after the
+ * call; calls that overlap in time need workspaces of their own.
+ * Contract as those entry points, plus ws 16-byte aligned. */
+int db_gemv_ws(const void* x, const void* g, const void* W, const void* W2,
+               const float* scale, const float* scale2, void* y, void* ws,
+               size_t ws_bytes, int B, int K, int N, float eps, int w_dtype,
+               void* stream);
+
 /* Split count the library picks for F4 when the caller has no preference:
- * about one (batch, kv-head, split) workgroup per CU of `cu_count` while
- * every split keeps at least eight 16-row tiles.  Replaces the fixed L/128 default and
+ * the one whose rounds of (batch, kv-head, split) workgroups on `cu_count`
+ * CUs are estimated to take the least time.  Replaces the fixed L/128 default and
  * DECODEBENCH_F4_SPLITS override of the reference harness
  * (validation/src/bench/bench_variant.cu:714-719). */
 int db_f4_default_splits(int B, int Hkv, int L, int cu_count);
@@ -168,7 +188,7 @@ int db_f4_splitkv(const void* q, const void* k, const void* v, void* o,
  * Contract as db_f4_splitkv, plus: the S' = min(S, ceil(L / 16)) splits must
  * fit, db_f4_workspace_bytes(B,Hq,Hkv,L,D,S') <= DB_F4_SCRATCH_BYTES, else
  * DB_ERR_INVALID (checked before any HIP call).  At the library's default
- * split count (about one workgroup per CU) that holds up to G = 8. */
+ * split count that holds up to G = 8. */
 int db_f4_splitkv_noalloc(const void* q, const void* k, const void* v, void* o,
                           int B, int Hq, int Hkv, int L, int D, int S,
                           float scale, void* stream);

@@ -57,6 +57,8 @@ extern "C" {
  *                         activations in LDS on the full grid; 0, the default,
  *                         off).  Either of these two set keeps one matrix at
  *                         K = 2048 and 4096 off the tile kernel
+ *  "gemv_splits"         (K splits of a db_gemv_ws call: 1 to 8 where its shape
+ *                         allows them; 0 automatic)
  *  "f4_launch"           (a call of F4 whose split merge runs in a second
  *                         launch makes only one of its two launches: 1 the
  *                         split kernel, 2 the merge, which then reads whatever

@@ -145,3 +145,68 @@ def test_tile_norm_keeps_precision_over_the_fp16_range(rows, dtype):
         x[3:9] = 0
     g = _randn(gen, K, std=1.0, mean=16.0)
     _check("f1", x, g, *_weights(gen, 1, N, K, dtype))
+
+
+# K split over workgroups: counts that divide the blocks and that do not, a
+# last split of one block, outputs that no quad or tile divides, more rows
+# than a pass, every mode and weight type.
+SPLIT_CASES = [
+    ("gemv", "f16", 9, 520, 1000, 2), ("gemv", "fp8", 17, 2064, 1023, 4),
+    ("f1", "f16", 24, 1336, 517, 3), ("f1", "fp8", 64, 4112, 2050, 8),
+    ("f2", "f16", 41, 1000, 700, 3), ("f2", "fp8", 12, 3088, 333, 4),
+    ("f2n", "f16", 16, 2600, 1021, 2), ("f2n", "fp8", 33, 4624, 512, 5),
+    ("gemv", "f16", 70, 3000, 4097, 4), ("f1", "f16", 130, 520, 260, 2),
+]
+
+
+@pytest.mark.parametrize("mode,dtype,B,K,N,S", SPLIT_CASES)
+def test_tile_splits(mode, dtype, B, K, N, S):
+    print(f"[tile-split] {mode} {dtype} B={B} K={K} N={N} S={S}", flush=True)
+    lib = ops.load_library()
+    gen = torch.Generator(device="cuda").manual_seed(B * 7919 + K + N)
+    x = _randn(gen, B, K)
+    g = _randn(gen, K, std=0.1, mean=1.0)
+    weights = _weights(gen, 2 if mode in ("f2", "f2n") else 1, N, K, dtype)
+    ops.tune("gemv_splits", S)
+    try:
+        assert lib.db_gemv_workspace_bytes(mode in ("f1", "f2n"), mode in ("f2", "f2n"), B, K, N,
+                                           dtype == "fp8") > 0
+        _check(mode, x, g, *weights)
+        # a call that brings its output takes one launch and allocates nothing
+        if mode == "gemv":
+            out = torch.empty(B, N, dtype=torch.float16, device="cuda")
+            held = torch.cuda.memory_stats()["allocation.all.allocated"]
+            ops.gemv(x, weights[0][0], w_scale=weights[1][0], out=out)
+            assert torch.cuda.memory_stats()["allocation.all.allocated"] == held
+            y = ops.gemv(x, weights[0][0], w_scale=weights[1][0])
+            assert (y.double() - out.double()).norm() <= 1e-3 * out.double().norm()
+    finally:
+        ops.tune("gemv_splits", 0)
+
+
+def test_tile_splits_capture_and_streams():
+    """Split calls captured into a graph (their workspaces come from its pool)
+    and on two streams at once."""
+    gen = torch.Generator(device="cuda").manual_seed(9)
+    x = _randn(gen, 20, 4096)
+    W = [_randn(gen, 1000, 4096, std=1 / 64) for _ in range(3)]
+    ops.tune("gemv_splits", 4)
+    try:
+        ref = [ops.gemv(x, w) for w in W]
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            ys = [ops.gemv(x, w) for w in W]
+        streams = [torch.cuda.Stream() for _ in range(2)]
+        for _ in range(4):
+            for st in streams:
+                st.wait_stream(torch.cuda.current_stream())
+            graph.replay()
+            side = []
+            for st in streams:
+                with torch.cuda.stream(st):
+                    side.append([ops.gemv(x, w) for w in W])
+            torch.cuda.synchronize()
+            for got in (ys, *side):
+                assert all(torch.equal(a, b) for a, b in zip(got, ref))
+    finally:
+        ops.tune("gemv_splits", 0)
