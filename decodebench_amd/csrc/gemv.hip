@@ -69,10 +69,12 @@ GemvFn gemv_pick_f1_two_rows(int u) {
 //    and the weights are few, so that the tile kernel's LDS staging and
 //    reduction show: [1024, 3072] at 4 rows 4.7 / 5.0, [2048, 1536] at 2
 //    rows 4.1 / 4.7 (2 rows of [8192, 8192] 24.3 / 23.5, F1 27.0 / 23.8).
-//  * The gate/up pair at K = 2048 and 4096, [14336, 4096]: 16-row passes to 16
-//    rows (fp16 40.0 / 39.8 at 16 rows, 38.2 / 39.3 at 4; e4m3 21.4 / 22.4 at
-//    4), the tile kernel above, where the passes read the weights again
-//    (fp16 at 32 and 64 rows 46.7 / 40.9 and 91.0 / 41.1, e4m3 61.9 / 29.4).
+//  * The gate/up pair at K = 2048 and 4096: 16-row passes to 11 rows ([14336,
+//    4096] fp16 38.2 / 38.8 at 4, e4m3 21.3 / 22.6), the tile kernel from 12
+//    (fp16 39.1 / 39.0 and 40.0 / 39.1 at 12 and 16, e4m3 [11008, 4096] 20.5 /
+//    19.2 and 20.2 / 18.9; fp16 at 32 and 64, where the passes read the weights
+//    again, 46.7 / 40.9 and 91.0 / 41.1, e4m3 61.9 / 29.4); with the RMSNorm
+//    from 17 (e4m3 [8192, 2048] at 16 rows 9.5 / 10.4, fp16 14.3 / 15.0).
 //  * F1 there: registers hold the activations up to 16 rows (fp16 [6144,
 //    4096] 11.3 / 11.5 at 4); above, fp16 takes tiles (24 rows 19.1 / 14.9,
 //    64 rows 28.8 / 21.5) except where one tile per CU leaves the statistic
@@ -96,7 +98,10 @@ bool tile_gemv(GemvMode mode, bool fp8, int B, int K, int N) {
     if (B == 2) return weights >= 40000000;
     return B >= 9 || weights >= (B <= 4 ? 10000000 : 4000000);
   }
-  if (pair) return B >= (t.gemv_pair_min_batch > 0 ? t.gemv_pair_min_batch : 17);
+  if (pair) {
+    const int from = mode == kGemvSwiGLU ? 12 : 17;
+    return B >= (t.gemv_pair_min_batch > 0 ? t.gemv_pair_min_batch : from);
+  }
   const bool one_tile = N <= 4096;
   if (K > 4096) {
     const bool forced = t.gemv_long_kc != 0 || t.gemv_long_gpw != 0 || t.gemv_long_stage != 0;

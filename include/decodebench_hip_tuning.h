@@ -45,7 +45,7 @@ extern "C" {
  *                         keeps plain rows longer than 4096 on that kernel
  *  "gemv_pair_min_batch" (batch rows from which the gate/up pair at K = 2048
  *                         and 4096 streams its activations on 16 x 16 tiles;
- *                         0 automatic, 17)
+ *                         0 automatic, 12, with the RMSNorm 17)
  *  "gemv_tile"           (batches of 2 rows and more: 1 always the streamed
  *                         16 x 16 tile kernel, 2 never; 0 automatic)
  *  "stream_waves"        (db_stream_read's waves per workgroup: 1, 2 or 4; 0
