@@ -486,6 +486,17 @@ def release_captured_workspaces() -> int:
     return n
 
 
+def _splits_for(workspace, B: int, Hq: int, Hkv: int, L: int, D: int, S: int, idx: int) -> int:
+    """The default split count ``S`` where the caller's workspace holds its
+    records, else that of a workgroup per CU and at least 8 tiles per split
+    (a caller may have sized the workspace for it)."""
+    held = workspace.numel() * workspace.element_size()
+    if held >= load_library().db_f4_workspace_bytes(B, Hq, Hkv, L, D, S):
+        return S
+    pairs, tiles = max(1, B * Hkv), -(-L // 16)
+    return max(1, min(S, -(-cu_count(idx) // pairs), max(1, tiles // 8), 256))
+
+
 def f4_flashdecode(q, K, V, scale: float | None = None, n_splits: int | None = None,
                    workspace=None, out=None):
     """F4: split-KV GQA decode attention with the log-sum-exp merge.
@@ -512,6 +523,8 @@ def f4_flashdecode(q, K, V, scale: float | None = None, n_splits: int | None = N
     lib = _lib or load_library()
     S = int(lib.db_f4_default_splits(B, Hkv, L, cu_count(idx))) if n_splits is None \
         else int(n_splits)
+    if workspace is not None and n_splits is None:
+        S = _splits_for(workspace, B, Hq, Hkv, L, D, S, idx)
     if workspace is None:
         workspace = f4_workspace(B, Hq, Hkv, L, D, S, idx)
     ws_ptr = workspace.data_ptr() if workspace is not None else None

@@ -80,3 +80,23 @@ def test_default_splits_attention(B, Hq, Hkv, L):
     # the scores' fp32 sums shift each exponent by at most 128 2^-24 |q||k| / sqrt(128)
     bound = 2 * u * mag + u * ref.abs() + 2.0 ** -13 * mag
     assert ((o - ref).abs() <= bound).all()
+
+
+@pytest.mark.gpu
+def test_a_workspace_for_one_workgroup_per_cu_still_serves():
+    """A caller's workspace sized for a workgroup per CU, where the default
+    now takes more splits; one too small for that is still refused."""
+    torch = pytest.importorskip("torch")
+    lib = ops.load_library()
+    B, Hq, Hkv, L = 12, 32, 8, 3001
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    q, K, V = (torch.randn(*s, generator=gen, device="cuda").half()
+               for s in ((B, Hq, 128), (B, Hkv, L, 128), (B, Hkv, L, 128)))
+    S0 = -(-ops.cu_count() // (B * Hkv))
+    assert ops.f4_default_splits(B, Hkv, L) > S0
+    need = lib.db_f4_workspace_bytes(B, Hq, Hkv, L, 128, S0)
+    ws = torch.zeros(need, dtype=torch.uint8, device="cuda")
+    assert torch.equal(ops.f4_flashdecode(q, K, V, workspace=ws),
+                       ops.f4_flashdecode(q, K, V, n_splits=S0))
+    with pytest.raises(ValueError, match="required"):
+        ops.f4_flashdecode(q, K, V, workspace=ws[:need - 256])
