@@ -76,13 +76,15 @@ GemvFn gemv_pick_f1_two_rows(int u) {
 //    again, 46.7 / 40.9 and 91.0 / 41.1, e4m3 61.9 / 29.4); with the RMSNorm
 //    from 17 (e4m3 [8192, 2048] at 16 rows 9.5 / 10.4, fp16 14.3 / 15.0).
 //  * F1 there: registers hold the activations up to 16 rows (fp16 [6144,
-//    4096] 11.3 / 11.5 at 4); above, fp16 takes tiles (24 rows 19.1 / 14.9,
-//    64 rows 28.8 / 21.5) except where one tile per CU leaves the statistic
-//    uncovered ([4096, 4096] at 32 rows 13.1 / 13.6), e4m3 stays (16.9 / 18).
+//    4096] 11.3 / 11.5 at 4); above, more than a tile per CU (fp16 at 24 and 64
+//    rows 18.6 / 14.2, 29.9 / 19.9, e4m3 11.7 / 11.5, 17.3 / 14.3), and one tile
+//    of fp16 at K = 4096 (32 and 64 rows 13.2 / 12.9, 20.3 / 14.8; e4m3 9.5 /
+//    9.6 and 13.0 / 13.3).
 //  * The plain projection: 3 rows and more (fp16 [4096, 4096] at 8, 24 and
 //    64 rows 8.9 / 8.6, 12.8 / 10.8, 19.8 / 14.6); at K = 2048 only with
 //    more than a tile per CU ([2048, 2048] at 16 rows 5.0 / 5.2); e4m3 with one
-//    tile per CU to 12 rows (6.8 / 6.2 at 8, 7.3 / 7.5 at 16).  To 3072
+//    tile per CU to 12 rows and from 17 (6.8 / 6.2 at 8, 7.3 / 7.5 at 16, 9.0 /
+//    8.3 at 24).  To 3072
 //    outputs (12 per CU) 16-row passes side by side read less of x ([1024,
 //    4096] at 4 and 32 rows 5.6 / 6.1, 6.1 / 7.1; F1 6.4 / 8.9 at 24), but for
 //    2048 and more above 32 rows.
@@ -109,10 +111,9 @@ bool tile_gemv(GemvMode mode, bool fp8, int B, int K, int N) {
   }
   if (t.gemv_xb != 0 || t.gemv_pass_grid != 0) return false;
   if (N <= 3072) return !fp8 && K == 4096 && N >= 2048 && B > 32;
-  if (mode == kGemvRmsNorm)
-    return !fp8 && K == 4096 && B >= 17 && (!one_tile || B <= 24 || B > 32);
+  if (mode == kGemvRmsNorm) return B >= 17 && (!one_tile || (!fp8 && K == 4096));
   if (K < 4096) return !one_tile && B >= 3;
-  return fp8 ? (B >= 3 && B <= 12) || (B >= 17 && !one_tile) : B >= 3;
+  return fp8 ? (B >= 3 && B <= 12) || B >= 17 : B >= 3;
 }
 
 // K splits of a call that has a workspace, 1 where one launch is as fast.

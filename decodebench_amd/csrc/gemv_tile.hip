@@ -68,17 +68,41 @@ hipError_t launch_gemv_tile(GemvMode mode, const void* x, const void* gamma, con
   a.part = static_cast<f4*>(ws);
   a.ssq = ws ? reinterpret_cast<float*>(static_cast<char*>(ws) + part_bytes(splits, pair, B, N))
              : nullptr;
+  // Passes of up to 64 batch rows, side by side on cu_count / passes workgroups
+  // each, so that the passes of a row range share an XCD's L2 copy of its
+  // weights.  Twice as many passes halve the x a CU reads and double its
+  // weights (from L2 for the second); one matrix takes them where the sum is no
+  // larger and the tiles per workgroup stay at 3 (at 4 where it falls by a
+  // fifth).  Measured on MI355X (us, one pass / two): F1 [6144, 4096] fp16 at 48
+  // and 64 rows 18.9 / 17.9, 20.0 / 17.7, e4m3 at 32 and 64 11.6 / 10.3, 17.2 /
+  // 13.7; e4m3 F1 [7168, 5120] at 64 20.6 / 18.6, but fp16 27.7 / 29.2.
+  const int per = pair ? 8 : 16;
+  auto tiles = [&](int passes, int* rows) {
+    // Outputs per workgroup: an even share of a workgroup per CU (of several
+    // rounds of them where a share would be more than 8 tiles).
+    const int slots = max(8, cu_count / passes / splits / 8 * 8);
+    const int rounds = (N + slots * per * kTileMaxTiles - 1) / (slots * per * kTileMaxTiles);
+    *rows = ((N + slots * rounds - 1) / (slots * rounds) + 3) / 4 * 4;
+    return (*rows + per - 1) / per;
+  };
+  int passes = (B + 8 * kTileMaxGroups - 1) / (8 * kTileMaxGroups);
+  int t = tiles(passes, &a.rows);
+  if (!pair && splits == 1 && B >= 17 * passes) {
+    const double weights = (double)N * K * (w.fp8 ? 1 : 2) / cu_count;
+    const double acts = 2.0 * B * K;
+    auto read = [&](int p) { return weights * p + acts / p; };
+    int rows = 0;
+    const int t2 = tiles(2 * passes, &rows);
+    const double ratio = read(2 * passes) / read(passes);
+    if ((t2 <= 3 && ratio <= 1.0) || (t2 <= 4 && ratio <= 0.8)) {
+      passes *= 2;
+      t = t2;
+      a.rows = rows;
+    }
+  }
   // Batch rows per pass: the fewest groups of 8 that hold an even share.
-  const int passes = (B + 8 * kTileMaxGroups - 1) / (8 * kTileMaxGroups);
   int nxg = ((B + passes - 1) / passes + 7) / 8;
   if (nxg == 5 || nxg == 7) ++nxg;
-  // Outputs per workgroup: an even share of a workgroup per CU (of several
-  // rounds of them where a share would be more than 8 tiles).
-  const int per = pair ? 8 : 16;
-  const int slots = max(8, cu_count / passes / splits / 8 * 8);
-  const int rounds = (N + slots * per * kTileMaxTiles - 1) / (slots * per * kTileMaxTiles);
-  a.rows = ((N + slots * rounds - 1) / (slots * rounds) + 3) / 4 * 4;
-  const int t = (a.rows + per - 1) / per;
   int grid = (N + a.rows - 1) / a.rows;
   if (passes > 1) grid = (grid + 7) / 8 * 8;
   const TileFn fn = w.fp8 ? (pair ? gemv_tile_pick_fp8_pair : gemv_tile_pick_fp8)(norm, t, nxg)
