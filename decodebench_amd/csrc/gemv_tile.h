@@ -26,8 +26,10 @@
 //    that neither side meets a bank twice.  No barrier: a wave's LDS accesses
 //    execute in order.  It costs 0.3 us of those 19.3.
 //  * Rows past N, batch rows past B and columns past K are loads past the
-//    buffer's range: they read zeros without touching memory, so tails need no
-//    masks (and an infinite weight meets no padding).
+//    buffer's range: they read zeros without touching memory, so the operands
+//    need no masks.  Where the groups of 8 batch rows are odd in number, the
+//    second half of the last 16-row operand is whatever is staged next (a weight
+//    block at times, whose bytes may be NaN as fp16): those sums are dropped.
 //  * Norm modes: operands are p = fp16(x * gamma) and the epilogue multiplies
 //    by 1 / rms, known only then.  The stage rounds fp16(x / rms) instead,
 //    whose range does not depend on x; so a wave first scales a row by a power
@@ -421,11 +423,14 @@ __global__ __launch_bounds__(tile_waves(T) * kWave) void gemv_tile_kernel(TileAr
       odd += off ? 1.0f : 0.0f;
     }
 #pragma unroll
-    for (int j = 0; j < T; ++j)
+    for (int bt = 0; bt < BT; ++bt) {
+      float fold = 0.0f;
 #pragma unroll
-      for (int bt = 0; bt < BT; ++bt)
+      for (int j = 0; j < T; ++j)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) odd = fmaf(acc[j][bt][i], 0.0f, odd);
+        for (int i = 0; i < 4; ++i) fold = fmaf(acc[j][bt][i], 0.0f, fold);
+      odd += 16 * bt + c16 < nb ? fold : 0.0f;  // no batch row, no sum
+    }
     const bool bad = !(odd == 0.0f);
     if (__builtin_expect(__any(bad), 0)) {
       set_scale(ss, n * KB);

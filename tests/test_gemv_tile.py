@@ -147,6 +147,27 @@ def test_tile_norm_keeps_precision_over_the_fp16_range(rows, dtype):
     _check("f1", x, g, *_weights(gen, 1, N, K, dtype))
 
 
+# Rows at both numbers of 8-row groups per 16-row tile; outputs for 8 waves of
+# one tile and 4 of more.
+NORM_CASES = [("f1", "f16", 4, 5120, 300), ("f1", "f16", 20, 3072, 4500),
+              ("f1", "fp8", 4, 3072, 300), ("f1", "fp8", 8, 8192, 4500),
+              ("f1", "fp8", 12, 3072, 300), ("f1", "fp8", 24, 3072, 4500),
+              ("f2n", "f16", 24, 4096, 300), ("f2n", "fp8", 8, 3072, 2500),
+              ("f2n", "fp8", 20, 4096, 2500)]
+
+
+@pytest.mark.parametrize("mode,dtype,B,K,N", NORM_CASES)
+def test_tile_norm_where_a_wave_scales_its_rows(mode, dtype, B, K, N):
+    """x around the mean squares at which a wave scales its rows, where its
+    first block says one thing and its columns another."""
+    gen = torch.Generator(device="cuda").manual_seed(B + K)
+    g = _randn(gen, K, std=0.1, mean=1.0)
+    weights = _weights(gen, 2 if mode == "f2n" else 1, N, K, dtype)
+    for std in (0.1, 0.12, 0.13, 0.14, 0.25, 100.0, 128.0, 200.0):
+        print(f"[tile-scale] {mode} {dtype} B={B} K={K} N={N} std={std}", flush=True)
+        _check(mode, _randn(gen, B, K, std=std), g, *weights)
+
+
 # K split over workgroups: counts that divide the blocks and that do not, a
 # last split of one block, outputs that no quad or tile divides, more rows
 # than a pass, every mode and weight type.
