@@ -36,7 +36,9 @@
 //    of two (exact) when its first block's mean square is outside [2^-6,
 //    2^14], and streams its columns a second time, scaled by their own mean
 //    square, when a sum is not finite or the first block was not
-//    representative (beyond 2^5 below or 2^8 above).  That second pass takes a
+//    representative (beyond 2^5 below or 2^8 above).  Always scaled: the first
+//    pass may have been scaled where the columns need none, or have overflowed
+//    in one product of a row of ordinary mean square.  That second pass takes a
 //    block at a time and the tests fold into one sum: as a second copy of the
 //    pipelined stream with branching tests they cost every call 3-8% (F1 fp16
 //    [7168, 5120] at 24 rows 18.4 us, 17.8 us now; e4m3 [6144, 4096] at 32 12.9, 11.4).
@@ -433,17 +435,18 @@ __global__ __launch_bounds__(tile_waves(T) * kWave) void gemv_tile_kernel(TileAr
     }
     const bool bad = !(odd == 0.0f);
     if (__builtin_expect(__any(bad), 0)) {
+      // Again with the columns' own scales, whatever they are: rare, and small
+      // code, a block at a time.
       set_scale(ss, n * KB);
-      if (scaled) {  // again, a block at a time: rare, and small code
-        clear();
-        for (int j = 0; j < n; ++j) {
-          load_x(0, j);
-          load_w(0, j);
-          stage(0);
-          product();
-        }
-        total_rows();
+      scaled = true;
+      clear();
+      for (int j = 0; j < n; ++j) {
+        load_x(0, j);
+        load_w(0, j);
+        stage(0);
+        product();
       }
+      total_rows();
     }
 #pragma unroll
     for (int q = 0; q < NXG; ++q)

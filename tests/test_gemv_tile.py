@@ -168,6 +168,38 @@ def test_tile_norm_where_a_wave_scales_its_rows(mode, dtype, B, K, N):
         _check(mode, _randn(gen, B, K, std=std), g, *weights)
 
 
+@pytest.mark.parametrize("mode,dtype,B,K,N", NORM_CASES)
+def test_tile_norm_where_one_block_is_unlike_the_others(mode, dtype, B, K, N):
+    """One block of columns far below or above the rest, at the first place, in
+    the middle and at the last: the block that some workgroup's wave starts at."""
+    gen = torch.Generator(device="cuda").manual_seed(B + K)
+    g = _randn(gen, K, std=0.1, mean=1.0)
+    weights = _weights(gen, 2 if mode == "f2n" else 1, N, K, dtype)
+    kb = 64 if dtype == "f16" else 128
+    for block in (0, K // kb // 2, K // kb - 1):
+        for e in (-12, -9, 9):
+            print(f"[tile-block] {mode} {dtype} B={B} K={K} N={N} block={block} e={e}", flush=True)
+            x = _randn(gen, B, K).float()
+            x[:, block * kb:(block + 1) * kb] *= 2.0 ** e
+            _check(mode, x.half(), g, *weights)
+
+
+@pytest.mark.parametrize("dtype", ["f16", "fp8"])
+@pytest.mark.parametrize("B", [4, 12])
+def test_tile_norm_where_one_product_leaves_fp16(B, dtype):
+    """Rows of ordinary mean square with one value whose product with gamma
+    overflows fp16, at the first columns, in the middle and at the last."""
+    gen = torch.Generator(device="cuda").manual_seed(B)
+    K, N = 5120, 4500
+    g = _randn(gen, K, std=1.0, mean=24.0)
+    weights = _weights(gen, 1, N, K, dtype)
+    for col in (3, K // 2 + 9, K - 1):
+        print(f"[tile-product] {dtype} B={B} col={col}", flush=True)
+        x = _randn(gen, B, K, std=60.0)
+        x[:, col] = 3000.0
+        _check("f1", x, g, *weights)
+
+
 # K split over workgroups: counts that divide the blocks and that do not, a
 # last split of one block, outputs that no quad or tile divides, more rows
 # than a pass, every mode and weight type.
