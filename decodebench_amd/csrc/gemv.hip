@@ -58,6 +58,16 @@ GemvFn gemv_pick_f1_two_rows(int u) {
   }
 }
 
+// Whether a knob of the calling thread keeps the call off the tile kernel, with
+// K splits or without.
+bool tile_barred(GemvMode mode, int B, int K, int N) {
+  const Tuning& t = tuning();
+  if (t.gemv_tile != 0) return t.gemv_tile == 2;
+  if (gemv_is_swiglu(mode) || !gemv_mfma_supported(mode, B, K, N)) return false;
+  return K > 4096 ? t.gemv_long_kc != 0 || t.gemv_long_gpw != 0 || t.gemv_long_stage != 0
+                  : t.gemv_xb != 0 || t.gemv_pass_grid != 0;
+}
+
 // Whether a batch of B rows takes the streamed tile kernel (gemv_tile.h)
 // rather than the MFMA kernels of gemv_mfma.hip or the VALU kernel below.
 // The lines lie where the two sides cross, measured on MI355X (graph back to
@@ -93,7 +103,8 @@ GemvFn gemv_pick_f1_two_rows(int u) {
 //    8.4 stays, and so do one-tile e4m3 calls above 48 rows (33.9 / 35.6).
 bool tile_gemv(GemvMode mode, bool fp8, int B, int K, int N) {
   const Tuning& t = tuning();
-  if (t.gemv_tile != 0) return t.gemv_tile == 1;
+  if (t.gemv_tile == 1) return true;
+  if (tile_barred(mode, B, K, N)) return false;
   const bool pair = gemv_is_swiglu(mode);
   const long weights = (long)N * K * (pair ? 2 : 1);
   if (!gemv_mfma_supported(mode, B, K, N)) {
@@ -105,11 +116,7 @@ bool tile_gemv(GemvMode mode, bool fp8, int B, int K, int N) {
     return B >= (t.gemv_pair_min_batch > 0 ? t.gemv_pair_min_batch : from);
   }
   const bool one_tile = N <= 4096;
-  if (K > 4096) {
-    const bool forced = t.gemv_long_kc != 0 || t.gemv_long_gpw != 0 || t.gemv_long_stage != 0;
-    return !forced && N > 2048 && !(fp8 && one_tile && B > 48);
-  }
-  if (t.gemv_xb != 0 || t.gemv_pass_grid != 0) return false;
+  if (K > 4096) return N > 2048 && !(fp8 && one_tile && B > 48);
   if (N <= 3072) return !fp8 && K == 4096 && N >= 2048 && B > 32;
   if (mode == kGemvRmsNorm) return B >= 17 && (!one_tile || (!fp8 && K == 4096));
   if (K < 4096) return !one_tile && B >= 3;
@@ -144,6 +151,7 @@ int tile_splits(GemvMode mode, bool fp8, int B, int K, int N, int cu_count) {
                       : ((N + slots - 1) / slots + (pair ? 7 : 15)) / (pair ? 8 : 16);
     return t <= kTileMaxTiles ? t : 0;
   };
+  if (tile_barred(mode, B, K, N)) return 1;
   if (forced > 0) return tiles(forced) > 0 ? forced : 1;
   const float x_kb = (float)B * (float)K * (2.0f / 1024.0f);
   if (B < 9 || K < 3072 || x_kb < 250.0f) return 1;

@@ -42,12 +42,14 @@ extern "C" {
  *                         automatic)
  *  "gemv_long_stage"     (its activations: 1 loaded as B operands, 2 staged
  *                         through LDS; 0 automatic).  Any of these three set
- *                         keeps plain rows longer than 4096 on that kernel
+ *                         keeps plain rows longer than 4096 that it takes (K
+ *                         a multiple of 2048) on that kernel, K splits or not
  *  "gemv_pair_min_batch" (batch rows from which the gate/up pair at K = 2048
  *                         and 4096 streams its activations on 16 x 16 tiles;
  *                         0 automatic, 12, with the RMSNorm 17)
  *  "gemv_tile"           (batches of 2 rows and more: 1 always the streamed
- *                         16 x 16 tile kernel, 2 never; 0 automatic)
+ *                         16 x 16 tile kernel, 2 never, K splits included; 0
+ *                         automatic)
  *  "stream_waves"        (db_stream_read's waves per workgroup: 1, 2 or 4; 0
  *                         is 4)
  *  "gemv_pass_grid"      (one weight matrix above 16 batch rows on MFMA:

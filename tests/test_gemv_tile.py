@@ -263,3 +263,28 @@ def test_tile_splits_capture_and_streams():
                 assert all(torch.equal(a, b) for a, b in zip(got, ref))
     finally:
         ops.tune("gemv_splits", 0)
+
+
+@pytest.mark.parametrize("knob,value", [("gemv_tile", 2), ("gemv_long_kc", 2),
+                                        ("gemv_long_gpw", 1), ("gemv_long_stage", 2)])
+@pytest.mark.parametrize("dtype", ["f16", "fp8"])
+def test_knobs_that_bar_the_tile_kernel_bar_its_splits(knob, value, dtype):
+    """Long plain rows that would split K: with the knob they get no workspace
+    and run the launch that a call with its own output runs."""
+    print(f"[tile-knob] {knob}={value} {dtype}", flush=True)
+    lib = ops.load_library()
+    gen = torch.Generator(device="cuda").manual_seed(11)
+    B, K, N = 32, 14336, 1000
+    x = _randn(gen, B, K)
+    W, s, W64 = _weights(gen, 1, N, K, dtype)
+    ops.tune("gemv_tile", 0)
+    assert lib.db_gemv_workspace_bytes(0, 0, B, K, N, dtype == "fp8") > 0
+    try:
+        ops.tune(knob, value)
+        assert lib.db_gemv_workspace_bytes(0, 0, B, K, N, dtype == "fp8") == 0
+        out = torch.empty(B, N, dtype=torch.float16, device="cuda")
+        ops.gemv(x, W[0], w_scale=s[0], out=out)
+        assert torch.equal(ops.gemv(x, W[0], w_scale=s[0]), out)
+        _check("gemv", x, None, W, s, W64)
+    finally:
+        ops.tune(knob, 0)

@@ -12,6 +12,7 @@ properties instead: split count invariance and agreement of batch rows with
 single-row launches.
 """
 
+import functools
 import math
 
 import numpy as np
@@ -239,7 +240,8 @@ def test_one_matrix_pass_shapes_agree():
 
 # --------------------------------------------------- long rows (MFMA, streamed x)
 # Plain GEMV with K a multiple of 2048 above 4096 -- the decode chain's down
-# projection, K = 14336 -- streams both operands in K chunks: batch tiles of
+# projection, K = 14336: the launch the library chooses, and the long-row
+# kernel, which streams both operands in K chunks: batch tiles of
 # 8, 16 and 32 rows in one pass, two passes above 32, N not a multiple of
 # the 8-row group, fewer groups than CUs, fp16 and e4m3 weights.
 LONG_CASES = [
@@ -262,15 +264,22 @@ def test_long_row_gemv_mfma_parity(dtype, B, K, N):
     W = randn(gen, (N, K), std=1.0 / math.sqrt(K))
     if dtype == "fp8":
         Wq, s = quantize_e4m3_rows(W)
-        y = ops.gemv(x.cuda(), Wq.cuda(), w_scale=s.cuda())
+        call = functools.partial(ops.gemv, x.cuda(), Wq.cuda(), w_scale=s.cuda())
         ref = stages.gemv_fp8(x, Wq, s)
         exact = cref.gemv_fp8_exact(x.numpy(), Wq.view(torch.uint8).numpy(), s.numpy())
     else:
-        y = ops.gemv(x.cuda(), W.cuda())
+        call = functools.partial(ops.gemv, x.cuda(), W.cuda())
         ref, exact = stages.gemv(x, W), cref.gemv_exact(x.numpy(), W.numpy())
-    torch.cuda.synchronize()
-    assert y.shape == (B, N)
-    assert_parity(y, ref, exact, F12_REL_L2, f"long {dtype} B={B} K={K} N={N}")
+    lib = ops.load_library()
+    for stage in (0, 2):  # 2: the long-row kernel as it runs by itself
+        assert lib.db_tune(b"gemv_long_stage", stage) == 0
+        try:
+            y = call()
+        finally:
+            lib.db_tune(b"gemv_long_stage", 0)
+        torch.cuda.synchronize()
+        assert y.shape == (B, N)
+        assert_parity(y, ref, exact, F12_REL_L2, f"long {dtype} B={B} K={K} N={N} stage={stage}")
 
 
 def test_long_row_gemv_launch_shapes_agree():
