@@ -99,8 +99,9 @@ bool tile_barred(GemvMode mode, int B, int K, int N) {
 //    4096] at 4 and 32 rows 5.6 / 6.1, 6.1 / 7.1; F1 6.4 / 8.9 at 24), but for
 //    2048 and more above 32 rows.
 //  * Its rows longer than 4096, above 8 outputs per CU: [4096, 14336] fp16
-//    at 16 rows 28.0 / 25.2, e4m3 at 8 rows 16.0 / 14.8; [1024, 8192] 7.3 /
-//    8.4 stays, and so do one-tile e4m3 calls above 48 rows (33.9 / 35.6).
+//    at 16 rows 28.0 / 25.2, e4m3 at 8 and 64 rows 16.0 / 14.8, 33.4 / 26.7;
+//    [1024, 8192] 7.3 / 8.4 stays, up to 64 rows ([1024, 14336] fp16 at 64 and 65
+//    21.3 / 21.5, 27.4 / 21.1; e4m3 [4096, 14336] at 128 64.0 / 36.2).
 bool tile_gemv(GemvMode mode, bool fp8, int B, int K, int N) {
   const Tuning& t = tuning();
   if (t.gemv_tile == 1) return true;
@@ -116,7 +117,7 @@ bool tile_gemv(GemvMode mode, bool fp8, int B, int K, int N) {
     return B >= (t.gemv_pair_min_batch > 0 ? t.gemv_pair_min_batch : from);
   }
   const bool one_tile = N <= 4096;
-  if (K > 4096) return N > 2048 && !(fp8 && one_tile && B > 48);
+  if (K > 4096) return N > 2048 || B > 64;
   if (N <= 3072) return !fp8 && K == 4096 && N >= 2048 && B > 32;
   if (mode == kGemvRmsNorm) return B >= 17 && (!one_tile || (!fp8 && K == 4096));
   if (K < 4096) return !one_tile && B >= 3;

@@ -265,6 +265,22 @@ def test_tile_splits_capture_and_streams():
         ops.tune("gemv_splits", 0)
 
 
+@pytest.mark.parametrize("dtype,B,K,N", [("fp8", 49, 8192, 4096), ("fp8", 64, 6144, 2057),
+                                         ("f16", 65, 8192, 260), ("fp8", 129, 10240, 1000)])
+def test_long_rows_of_many_batch_rows_take_the_tile_kernel(dtype, B, K, N):
+    """Into a given output (one launch): the bits of the forced tile kernel."""
+    print(f"[tile-long] {dtype} B={B} K={K} N={N}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(B * 7919 + K + N)
+    x = _randn(gen, B, K)
+    W, s, W64 = _weights(gen, 1, N, K, dtype)
+    out = [torch.empty(B, N, dtype=torch.float16, device="cuda") for _ in range(2)]
+    ops.gemv(x, W[0], w_scale=s[0], out=out[0])
+    ops.tune("gemv_tile", 0)
+    ops.gemv(x, W[0], w_scale=s[0], out=out[1])
+    assert torch.equal(*out)
+    _check("gemv", x, None, W, s, W64)
+
+
 @pytest.mark.parametrize("knob,value", [("gemv_tile", 2), ("gemv_long_kc", 2),
                                         ("gemv_long_gpw", 1), ("gemv_long_stage", 2)])
 @pytest.mark.parametrize("dtype", ["f16", "fp8"])
