@@ -132,20 +132,28 @@ bool tile_gemv(GemvMode mode, bool fp8, int B, int K, int N) {
 // partial sums per output and a second launch, about 1.5 us and 0.7 us per
 // tile (1.4 for the pair) against the 52 GB/s at which a CU reads x between
 // weights.  Measured on MI355X (us, one launch / 4 splits): fp16 [4096, 14336] at
-// 12, 24 and 64 rows 23.2 / 23.1, 30.3 / 24.2, 44.3 / 28.8, e4m3 at 64 34.1 /
-// 23.7; [4096, 11008] at 12 and 41 rows 18.7 / 19.0, 27.8 / 21.6; [1024, 4096]
-// at 64 11.5 / 8.3; [4096, 4096] at 24 and 64 10.5 / 11.2, 14.7 / 13.3; pair
-// [2048, 8192] at 24 and 64 17.3 / 17.9, 24.9 / 21.4.  2 and 8 splits were
-// behind 4, and 3 ahead where they fill the CUs with 4 tiles and 4 splits take
-// 5 ([5120, 5120] at 41 rows 19.8 / 16.4 / 17.0); more than 4 tiles gained
-// nothing (e4m3 F1 [7168, 5120] at 64 rows 20.7 / 22.8), nor did short rows
-// ([2048, 2048] at 64 7.3 / 8.5).
+// 12, 24 and 64 rows 23.2 / 23.1, 30.3 / 24.2, 42.7 / 28.7, e4m3 at 64 26.7 /
+// 21.6; [4096, 11008] at 12 and 41 rows 18.7 / 19.0, 26.0 / 20.3; [4096, 4096]
+// at 24 and 64 10.5 / 11.2, 13.3 / 12.8; pair [2048, 8192] at 24 and 64 17.3 /
+// 17.9, 24.8 / 19.9.  2 and 8 splits were behind 4, and 3 ahead where they fill
+// the CUs with 4 tiles and 4 splits take 5 ([5120, 5120] at 41 rows 19.8 / 16.4
+// / 17.0); more than 4 tiles gained nothing (e4m3 F1 [7168, 5120] at 64 rows
+// 20.7 / 22.8), nor did short rows ([2048, 2048] at 64 7.3 / 8.5).
+// Above 64 rows the passes share the CUs, as in launch_gemv_tile: 65 rows of
+// 4096 outputs take 8 tiles per workgroup, not 4, at about 1.1 us each.  Long
+// rows still gain (fp16 [4096, 11008] at 65 and 128 rows 37.6 / 31.5, 40.5 /
+// 32.5; e4m3 [1024, 14336] at 129 20.8 / 17.2), 4096 columns do not ([4096, 4096]
+// at 65 and 128 13.7 / 16.1, 15.8 / 20.1), and neither does a count whose
+// workgroups take another round ([4096, 4096] at 256 21.1 / 32.1, [5120, 5120]
+// F1 34.7 / 61.8; of 24 shapes at 129 to 1024 rows 5 lost by it, most [4096,
+// 14336] at 256 rows, 83 / 69).  That bounds the workspace to 8 MB at any batch.
 int tile_splits(GemvMode mode, bool fp8, int B, int K, int N, int cu_count) {
   const bool pair = gemv_is_swiglu(mode);
   const int forced = tuning().gemv_splits;
-  // Tiles per workgroup with S splits, 0 where there are too few columns.
-  auto tiles = [&](int S) {
-    const int slots = cu_count / S / 8 * 8;
+  // Tiles per workgroup with S splits, 0 where there are too few columns or
+  // the workgroups would take another round.
+  auto tiles = [&](int S, int passes) {
+    const int slots = cu_count / passes / S / 8 * 8;
     const int blocks = (K + (fp8 ? 127 : 63)) / (fp8 ? 128 : 64);
     const int t = slots < 8 || blocks < 4 * S
                       ? 0
@@ -153,15 +161,19 @@ int tile_splits(GemvMode mode, bool fp8, int B, int K, int N, int cu_count) {
     return t <= kTileMaxTiles ? t : 0;
   };
   if (tile_barred(mode, B, K, N)) return 1;
-  if (forced > 0) return tiles(forced) > 0 ? forced : 1;
-  const float x_kb = (float)B * (float)K * (2.0f / 1024.0f);
+  if (forced > 0) return tiles(forced, 1) > 0 ? forced : 1;
+  const int passes = tile_passes(B);
+  const int rows = min(B, 8 * tile_groups(B, passes));
+  const float x_kb = (float)rows * (float)K * (2.0f / 1024.0f);
   if (B < 9 || K < 3072 || x_kb < 250.0f) return 1;
   if (K <= 4096 && !tile_gemv(mode, fp8, B, K, N)) return 1;
-  const int S = tiles(4) > 4 && tiles(3) > 0 && tiles(3) <= 4 ? 3 : 4;
-  const int t = tiles(S);
-  if (t == 0 || t > 4) return 1;
+  const int t3 = tiles(3, passes), t4 = tiles(4, passes);
+  const int S = t4 > 4 && t3 > 0 && t3 <= 4 ? 3 : 4;
+  const int t = S == 3 ? t3 : t4;
+  if (t == 0 || (passes == 1 && t > 4)) return 1;
+  const float per_tile = t > 4 ? 1.1f : pair ? 1.4f : 0.7f;
   const float gain = x_kb * (1.0f - 1.0f / (float)S) / 52.0f;
-  return gain > 2.0f + (pair ? 1.4f : 0.7f) * (float)t ? S : 1;
+  return gain > 2.0f + per_tile * (float)t ? S : 1;
 }
 
 }  // namespace

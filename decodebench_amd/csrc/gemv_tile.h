@@ -77,6 +77,13 @@ using TileFn = void (*)(TileArgs);
 // tiles of 16 (T of them).
 constexpr int kTileMaxTiles = 8;
 constexpr int kTileMaxGroups = 8;
+// Passes of a batch, and the groups of a workgroup of one of passes side by
+// side: the fewest that hold an even share, of the counts there are kernels for.
+inline int tile_passes(int B) { return (B + 8 * kTileMaxGroups - 1) / (8 * kTileMaxGroups); }
+inline int tile_groups(int B, int passes) {
+  const int g = ((B + passes - 1) / passes + 7) / 8;
+  return g == 5 || g == 7 ? g + 1 : g;
+}
 constexpr int tile_lines(bool fp8) { return fp8 ? 2 : 1; }  // x lines per block
 // Waves per workgroup: 8 waves of one tile, 4 of more (2 tiles at 4 rows: 10.5
 // us with 4 waves, 11.3 with 8; 7 tiles at 16 rows 37.3 against 38.7).

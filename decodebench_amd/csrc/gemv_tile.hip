@@ -85,7 +85,7 @@ hipError_t launch_gemv_tile(GemvMode mode, const void* x, const void* gamma, con
     *rows = ((N + slots * rounds - 1) / (slots * rounds) + 3) / 4 * 4;
     return (*rows + per - 1) / per;
   };
-  int passes = (B + 8 * kTileMaxGroups - 1) / (8 * kTileMaxGroups);
+  int passes = tile_passes(B);
   int t = tiles(passes, &a.rows);
   if (!pair && splits == 1 && B >= 17 * passes) {
     const double weights = (double)N * K * (w.fp8 ? 1 : 2) / cu_count;
@@ -100,9 +100,7 @@ hipError_t launch_gemv_tile(GemvMode mode, const void* x, const void* gamma, con
       a.rows = rows;
     }
   }
-  // Batch rows per pass: the fewest groups of 8 that hold an even share.
-  int nxg = ((B + passes - 1) / passes + 7) / 8;
-  if (nxg == 5 || nxg == 7) ++nxg;
+  const int nxg = tile_groups(B, passes);
   int grid = (N + a.rows - 1) / a.rows;
   if (passes > 1) grid = (grid + 7) / 8 * 8;
   const TileFn fn = w.fp8 ? (pair ? gemv_tile_pick_fp8_pair : gemv_tile_pick_fp8)(norm, t, nxg)

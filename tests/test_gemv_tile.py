@@ -304,3 +304,40 @@ def test_knobs_that_bar_the_tile_kernel_bar_its_splits(knob, value, dtype):
         _check("gemv", x, None, W, s, W64)
     finally:
         ops.tune(knob, 0)
+
+
+def test_split_workspace_is_bounded_at_any_batch():
+    """One round of workgroups: 256 of up to 8 tiles of 16 outputs, 64 batch
+    rows and 4 bytes, 8 MB, and the sums of x^2 (8 splits x 4 bytes a row)."""
+    lib = ops.load_library()
+    ops.tune("gemv_tile", 0)
+    split = 0
+    for B in (9, 40, 64, 65, 128, 129, 256, 600, 8192, 65536):
+        for K in (3072, 4096, 5120, 8192, 14336):
+            for N in (512, 1024, 3000, 4096, 5120, 14336):
+                for norm, pair in ((0, 0), (1, 0), (0, 1), (1, 1)):
+                    for dt in (0, 1):
+                        n = lib.db_gemv_workspace_bytes(norm, pair, B, K, N, dt)
+                        assert n <= (8 << 20) + 32 * B, (B, K, N, norm, pair, dt)
+                        split += n > 0
+    assert split > 0
+
+
+# More rows than a pass: splits of one round of workgroups, shapes that would
+# take two rounds (no splits), and long rows that no longer split.
+@pytest.mark.parametrize("mode,dtype,B,K,N,split", [
+    ("gemv", "f16", 65, 11008, 2050, True), ("gemv", "fp8", 129, 14336, 1024, True),
+    ("f1", "f16", 100, 8192, 2047, True), ("f2n", "f16", 130, 8192, 1021, True),
+    ("gemv", "f16", 65, 4096, 4096, False), ("gemv", "fp8", 200, 8192, 4095, False),
+    ("f2", "f16", 129, 8192, 2048, False), ("gemv", "f16", 257, 6144, 2040, False),
+])
+def test_automatic_splits_above_one_pass(mode, dtype, B, K, N, split):
+    print(f"[tile-rows] {mode} {dtype} B={B} K={K} N={N}", flush=True)
+    lib = ops.load_library()
+    ops.tune("gemv_tile", 0)
+    assert (lib.db_gemv_workspace_bytes(mode in ("f1", "f2n"), mode in ("f2", "f2n"), B, K, N,
+                                        dtype == "fp8") > 0) == split
+    gen = torch.Generator(device="cuda").manual_seed(B * 7919 + K + N)
+    x = _randn(gen, B, K)
+    g = _randn(gen, K, std=0.1, mean=1.0)
+    _check(mode, x, g, *_weights(gen, 2 if mode in ("f2", "f2n") else 1, N, K, dtype))
