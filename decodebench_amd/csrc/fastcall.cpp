@@ -138,11 +138,16 @@ PyObject* gemv_op(PyObject* xo, PyObject* go, PyObject* w0o, PyObject* w1o, PyOb
   void* yp = y.data_ptr();
   const int b = (int)B, k = (int)K, n = (int)N;
   // K split over workgroups, in a workspace that the allocator takes back in
-  // stream order after this call.
+  // stream order after this call; one launch where there is no room for it.
   at::Tensor ws;
-  const size_t bytes = b > 8 ? abi.gemv_workspace_bytes(g != nullptr, w1 != nullptr, b, k, n, dtype) : 0;
-  if (bytes > 0)
-    ws = at::empty({(int64_t)bytes}, at::TensorOptions().dtype(at::kByte).device(y.device()));
+  size_t bytes = b > 8 ? abi.gemv_workspace_bytes(g != nullptr, w1 != nullptr, b, k, n, dtype) : 0;
+  if (bytes > 0) {
+    try {
+      ws = at::empty({(int64_t)bytes}, at::TensorOptions().dtype(at::kByte).device(y.device()));
+    } catch (const c10::OutOfMemoryError&) {
+      bytes = 0;
+    }
+  }
   void* wsp = bytes > 0 ? ws.data_ptr() : nullptr;
   int rc;
   Py_BEGIN_ALLOW_THREADS

@@ -308,14 +308,18 @@ def _split_launch(out, x, g, W, W2, s, s2, y, B: int, K: int, N: int, eps: float
     """Launch a GEMV op with K split over workgroups, in a workspace from
     torch's allocator, where the library would (``db_gemv_workspace_bytes``).
     Returns whether it did; a call with its own ``out`` allocates nothing, and
-    a refused one is left to the entry point without a workspace."""
+    one that is refused or has no room for the workspace is left to the entry
+    point without one."""
     torch, lib = _torch, _lib or load_library()
     if out is not None or B < 9 or torch.cuda.current_device() != idx:
         return False
     nbytes = lib.db_gemv_workspace_bytes(g is not None, W2 is not None, B, K, N, dt)
     if nbytes == 0:
         return False
-    ws = torch.empty(nbytes, dtype=torch.uint8, device=y.device)
+    try:
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=y.device)
+    except torch.cuda.OutOfMemoryError:
+        return False
     return lib.db_gemv_ws(x, g, W, W2, s, s2, y.data_ptr(), ws.data_ptr(), nbytes, B, K, N, eps,
                           dt, _raw_stream(idx)) == DB_OK
 

@@ -341,3 +341,31 @@ def test_automatic_splits_above_one_pass(mode, dtype, B, K, N, split):
     x = _randn(gen, B, K)
     g = _randn(gen, K, std=0.1, mean=1.0)
     _check(mode, x, g, *_weights(gen, 2 if mode in ("f2", "f2n") else 1, N, K, dtype))
+
+
+def test_split_call_without_room_for_its_workspace_takes_one_launch(monkeypatch):
+    """Memory for the output but not for the partial sums: the call still
+    answers, through either call path."""
+    ops.tune("gemv_tile", 0)
+    B, K, N = 40, 11008, 4096
+    gen = torch.Generator(device="cuda").manual_seed(2)
+    torch.cuda.empty_cache()
+    # made in place: no segment with a hole that a workspace fits in
+    x = torch.empty(B, K, dtype=torch.float16, device="cuda").normal_(generator=gen)
+    W = torch.empty(N, K, dtype=torch.float16, device="cuda").normal_(0, K ** -0.5, generator=gen)
+    assert ops.load_library().db_gemv_workspace_bytes(0, 0, B, K, N, 0) > 1 << 20
+    ref = ops.gemv(x, W, out=torch.empty(B, N, dtype=torch.float16, device="cuda"))
+    assert not torch.equal(ops.gemv(x, W), ref)  # split, with memory
+    total = torch.cuda.get_device_properties(0).total_memory
+    for fast in (ops._fast, None):
+        monkeypatch.setattr(ops, "_fast", fast)
+        torch.cuda.empty_cache()
+        y = torch.empty(B, N, dtype=torch.float16, device="cuda")
+        del y  # a cached block for the output
+        torch.cuda.set_per_process_memory_fraction(
+            (torch.cuda.memory_reserved() + (1 << 20)) / total)
+        try:
+            y = ops.gemv(x, W)
+        finally:
+            torch.cuda.set_per_process_memory_fraction(1.0)
+        assert torch.equal(y, ref)
