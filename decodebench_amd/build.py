@@ -73,14 +73,25 @@ def _compile(src: Path) -> Path:
     return obj
 
 
+def _fast_stale() -> bool:
+    """Whether the native call path is missing, older than its sources or built
+    for another torch or Python (which its file holds as a text)."""
+    from decodebench_amd.ops import fast_built_for
+
+    return _stale(FAST_LIB, FAST_SRC) or fast_built_for().encode() not in FAST_LIB.read_bytes()
+
+
 def _compile_fast(src: Path) -> Path:
     import torch
+
+    from decodebench_amd.ops import fast_built_for
 
     root = Path(torch.__file__).resolve().parent
     tmp = FAST_LIB.with_suffix(".so.tmp")
     abi = int(getattr(torch._C, "_GLIBCXX_USE_CXX11_ABI", True))
     cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared",
-           f"-D_GLIBCXX_USE_CXX11_ABI={abi}", f"-I{sysconfig.get_paths()['include']}",
+           f"-D_GLIBCXX_USE_CXX11_ABI={abi}", f'-DDB_BUILT_FOR="{fast_built_for()}"',
+           f"-I{sysconfig.get_paths()['include']}",
            f"-I{root / 'include'}", f"-I{root / 'include/torch/csrc/api/include'}", str(src),
            "-o", str(tmp), f"-L{root / 'lib'}", "-ltorch_python", "-ltorch_cpu", "-lc10"]
     res = subprocess.run(cmd, capture_output=True, text=True)
@@ -98,7 +109,7 @@ def build(force: bool = False, verbose: bool = True) -> Path:
     srcs = _sources()
     todo = [s for s in srcs if force or _stale(BUILD / (s.stem + ".o"), s)]
     jobs = [(_compile, s) for s in todo]
-    if force or _stale(FAST_LIB, FAST_SRC):
+    if force or _fast_stale():
         jobs.insert(0, (_compile_fast, FAST_SRC))
     if jobs:
         workers = min(len(jobs), max(1, (os.cpu_count() or 2)))

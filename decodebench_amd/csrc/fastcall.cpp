@@ -23,6 +23,10 @@
 
 #include "../../include/decodebench_hip.h"
 
+#ifndef DB_BUILT_FOR
+#error "build with decodebench_amd.build, which defines DB_BUILT_FOR"
+#endif
+
 namespace {
 
 struct Abi {
@@ -317,4 +321,10 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_fastcall", nullptr, -1, methods,
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__fastcall(void) { return PyModule_Create(&module); }
+// built_for names the torch and the Python whose object layouts this module
+// holds; its functions are only called where both are the running ones.
+PyMODINIT_FUNC PyInit__fastcall(void) {
+  PyObject* m = PyModule_Create(&module);
+  if (m && PyModule_AddStringConstant(m, "built_for", DB_BUILT_FOR) < 0) Py_CLEAR(m);
+  return m;
+}

@@ -25,6 +25,7 @@ from __future__ import annotations
 
 import ctypes as C
 import math
+import sys
 import threading
 from pathlib import Path
 
@@ -99,6 +100,13 @@ def load_library():
         return lib
 
 
+def fast_built_for() -> str:
+    """The torch and the Python that a ``_fastcall`` module has to be built for
+    to be used: it holds their object layouts, which an import does not check."""
+    torch = _torch or _torch_mod()
+    return f"torch {torch.__version__}, {sys.implementation.cache_tag}"
+
+
 def _load_fast(lib) -> None:
     """Load the native call path and hand it the library's entry points."""
     global _fast
@@ -114,7 +122,9 @@ def _load_fast(lib) -> None:
     try:
         mod = importlib.util.module_from_spec(spec)
         loader.exec_module(mod)
-    except ImportError:  # built against another torch
+    except ImportError:  # built against another torch whose symbols differ
+        return
+    if getattr(mod, "built_for", None) != fast_built_for():
         return
     entry = tuple(C.cast(getattr(lib, name), C.c_void_p).value for name in (
         "db_f1_rmsnorm_gemv", "db_f2_gateup_swiglu", "db_f2_rmsnorm_gateup_swiglu", "db_gemv",

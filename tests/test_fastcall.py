@@ -62,6 +62,18 @@ def test_refusals_are_the_python_steps_own(steps):
         assert isinstance(fast, tuple) and fast == slow
 
 
+def test_a_module_built_for_another_torch_is_not_used(monkeypatch):
+    """Its symbols may resolve all the same; its object layouts need not fit."""
+    _load()
+    from decodebench_amd import build
+
+    assert not build._fast_stale()
+    monkeypatch.setattr(ops, "_fast", None)
+    monkeypatch.setattr(torch, "__version__", "0.0")
+    ops._load_fast(ops.load_library())
+    assert ops._fast is None and build._fast_stale()
+
+
 def _inputs():
     gen = torch.Generator(device="cuda").manual_seed(3)
 
