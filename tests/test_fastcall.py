@@ -74,6 +74,26 @@ def test_a_module_built_for_another_torch_is_not_used(monkeypatch):
     assert ops._fast is None and build._fast_stale()
 
 
+def test_the_library_is_built_where_the_call_path_is_not(monkeypatch, tmp_path):
+    """No g++, headers or torch: a warning, the library, and no stale module."""
+    from decodebench_amd import build
+
+    lib, old = tmp_path / "lib.so", tmp_path / "_fastcall.so"
+    lib.write_bytes(b"linked")
+    old.write_bytes(b"stale")
+
+    def no_compiler(cmd, **kw):
+        raise FileNotFoundError(cmd[0])
+
+    monkeypatch.setattr(build, "_sources", list)
+    monkeypatch.setattr(build, "LIB", lib)
+    monkeypatch.setattr(build, "FAST_LIB", old)
+    monkeypatch.setattr(build.subprocess, "run", no_compiler)
+    with pytest.warns(UserWarning, match="native call path"):
+        assert build.build(verbose=False) == lib
+    assert not old.exists()
+
+
 def _inputs():
     gen = torch.Generator(device="cuda").manual_seed(3)
 
