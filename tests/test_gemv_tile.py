@@ -349,22 +349,24 @@ def test_split_call_without_room_for_its_workspace_takes_one_launch(monkeypatch)
     ops.tune("gemv_tile", 0)
     B, K, N = 40, 11008, 4096
     gen = torch.Generator(device="cuda").manual_seed(2)
-    torch.cuda.empty_cache()
-    # made in place: no segment with a hole that a workspace fits in
-    x = torch.empty(B, K, dtype=torch.float16, device="cuda").normal_(generator=gen)
-    W = torch.empty(N, K, dtype=torch.float16, device="cuda").normal_(0, K ** -0.5, generator=gen)
-    assert ops.load_library().db_gemv_workspace_bytes(0, 0, B, K, N, 0) > 1 << 20
+    x, W = _randn(gen, B, K), _randn(gen, N, K, std=K ** -0.5)
+    nbytes = ops.load_library().db_gemv_workspace_bytes(0, 0, B, K, N, 0)
+    assert nbytes > 1 << 20
     ref = ops.gemv(x, W, out=torch.empty(B, N, dtype=torch.float16, device="cuda"))
     assert not torch.equal(ops.gemv(x, W), ref)  # split, with memory
     total = torch.cuda.get_device_properties(0).total_memory
     for fast in (ops._fast, None):
         monkeypatch.setattr(ops, "_fast", fast)
-        torch.cuda.empty_cache()
         y = torch.empty(B, N, dtype=torch.float16, device="cuda")
-        del y  # a cached block for the output
+        torch.cuda.empty_cache()
         torch.cuda.set_per_process_memory_fraction(
             (torch.cuda.memory_reserved() + (1 << 20)) / total)
+        full = []
         try:
+            with pytest.raises(torch.cuda.OutOfMemoryError):
+                while True:  # every block that the workspace would fit in
+                    full.append(torch.empty(nbytes, dtype=torch.uint8, device="cuda"))
+            del y  # room for the output
             y = ops.gemv(x, W)
         finally:
             torch.cuda.set_per_process_memory_fraction(1.0)
