@@ -34,7 +34,7 @@
 //    by 1 / rms, known only then.  The stage rounds fp16(x / rms) instead,
 //    whose range does not depend on x; so a wave first scales a row by a power
 //    of two (exact) when its first block's mean square is outside [2^-6,
-//    2^14], and streams its columns a second time, scaled by their own mean
+//    2^14] or gamma's is below 2^-20, and streams its columns a second time, scaled by their own mean
 //    square, when a sum is not finite or the first block was not
 //    representative (beyond 2^5 below or 2^8 above).  Always scaled: the first
 //    pass may have been scaled where the columns need none, or have overflowed
@@ -336,13 +336,13 @@ __global__ __launch_bounds__(tile_waves(T) * kWave) void gemv_tile_kernel(TileAr
   };
   // NORM: scale every row by the power of two that brings its mean square
   // (sum sq over cols columns) near 1, unless every row's is in the range that
-  // needs none.
-  auto set_scale = [&](const float (&sq)[NXG], int cols) {
+  // needs none and gamma is not so small that its products leave fp16's.
+  auto set_scale = [&](const float (&sq)[NXG], int cols, bool small_gamma) {
     bool need = false;
 #pragma unroll
     for (int q = 0; q < NXG; ++q) {
       const float ms = sq[q] / (float)cols;
-      need = need || (ms > 0.0f && (ms < 0x1p-6f || ms > 0x1p14f));
+      need = need || (ms > 0.0f && (ms < 0x1p-6f || ms > 0x1p14f || small_gamma));
       const int e = ms > 0.0f ? (1 - __builtin_amdgcn_frexp_expf(ms)) >> 1 : 0;
       const _Float16 f = (_Float16)__builtin_amdgcn_ldexpf(1.0f, max(-16, min(15, e)));
       scale[q] = h2{f, f};
@@ -369,7 +369,9 @@ __global__ __launch_bounds__(tile_waves(T) * kWave) void gemv_tile_kernel(TileAr
     for (int d = 0; d < DEPTH; ++d) load_w(d, d);
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (NORM) {
-      float sq[NXG];
+      float sq[NXG], gg = 0.0f;
+#pragma unroll
+      for (int l = 0; l < LINES; ++l) gg = dot8(gs[0][l], gs[0][l], gg);
 #pragma unroll
       for (int q = 0; q < NXG; ++q) {
         float v = 0.0f;
@@ -377,7 +379,7 @@ __global__ __launch_bounds__(tile_waves(T) * kWave) void gemv_tile_kernel(TileAr
         for (int l = 0; l < LINES; ++l) v = dot8(xs[0][q * LINES + l], xs[0][q * LINES + l], v);
         sq[q] = row8(v);
       }
-      set_scale(sq, KB);
+      set_scale(sq, KB, row8(gg) < KB * 0x1p-20f);
     }
     int j = 0;
     for (; j + 2 * DEPTH <= n; j += DEPTH) {
@@ -444,7 +446,7 @@ __global__ __launch_bounds__(tile_waves(T) * kWave) void gemv_tile_kernel(TileAr
     if (__builtin_expect(__any(bad), 0)) {
       // Again with the columns' own scales, whatever they are: rare, and small
       // code, a block at a time.
-      set_scale(ss, n * KB);
+      set_scale(ss, n * KB, false);
       scaled = true;
       clear();
       for (int j = 0; j < n; ++j) {

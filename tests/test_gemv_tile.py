@@ -200,6 +200,29 @@ def test_tile_norm_where_one_product_leaves_fp16(B, dtype):
         _check("f1", x, g, *weights)
 
 
+@pytest.mark.parametrize("dtype", ["f16", "fp8"])
+@pytest.mark.parametrize("std", [0.126, 0.25, 1.0])
+def test_tile_norm_keeps_precision_under_a_small_gamma(std, dtype):
+    """gamma of 2^-13: its product with a normalised row, of which fp16 keeps 11
+    bits, less what the subnormals below 2^-14 lose.  Relative error, of the
+    2-norms: 2^-11 x 0.41 for each of two roundings (the mean over a binade),
+    2^-24 / sqrt(12) of 2^-13 for the subnormals: 3.2e-4; 4.5e-4 allows for the
+    stage's third rounding.  Without a scale x of 0.25 gives 5.9e-4."""
+    print(f"[tile-gamma] std={std} {dtype}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(6)
+    B, K, N = 12, 3072, 1000
+    x = _randn(gen, B, K, std=std)
+    g = ((torch.randn(K, generator=gen, device="cuda") * 0.1 + 1) * 2.0 ** -13).half()
+    w = _randn(gen, N, K, std=8 * K ** -0.5)
+    w, s = quantize_e4m3_rows(w) if dtype == "fp8" else (w, None)
+    w64 = (dequantize_e4m3_rows(w, s) if dtype == "fp8" else w).double()
+    p = x.double()
+    p = p * torch.rsqrt(p.square().mean(-1, keepdim=True) + 1e-6) * g.double()
+    ref = p @ w64.t().contiguous()
+    err = (ops.f1_rmsnorm_gemv(x, g, w, w_scale=s).double() - ref).norm() / ref.norm()
+    assert err <= 4.5e-4, f"{err.item():.2e}"
+
+
 # K split over workgroups: counts that divide the blocks and that do not, a
 # last split of one block, outputs that no quad or tile divides, more rows
 # than a pass, every mode and weight type.
