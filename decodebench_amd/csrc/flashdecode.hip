@@ -780,8 +780,8 @@ size_t f4_workspace_bytes(int B, int Hq, int Hkv, int S, int D) {
 // longest split: about 0.3 us per 16-row tile while the whole chip streams,
 // 1.6 us more per further round, and the merge (1.5 us to 8 splits, which one
 // thread per output merges, 2.9 us above, 3.5 where 4 waves take a second
-// chunk of splits).  So a count that just spills over
-// into another round is avoided (20 x 8 pairs at L = 3001 with 2 splits, 1.25
+// chunk of splits; 3.2 and 3.8 in a launch of its own, however few).  So a count
+// that just spills over into another round is avoided (20 x 8 pairs at L = 3001 with 2 splits, 1.25
 // rounds, 54.7 us; with 3, 1.9 rounds, 43.9), and so is one round of few
 // workgroups (12 x 8 pairs: 3 splits 40.7, 2 splits 34.4, 5 splits 31.2).
 // Measured on MI355X (graph back to back, us, a workgroup per CU rounded up /
@@ -789,6 +789,9 @@ size_t f4_workspace_bytes(int B, int Hq, int Hkv, int S, int D) {
 // 33.8, 32.9 / 24.7; B = 10, 24, 36, 40 at L = 3001 30.8 / 24.8, 61.9 / 50.6,
 // 103.8 / 79.9, 106.2 / 82.9; B = 1 at L = 300 and 3001 6.4 / 5.3, 8.2 / 7.9;
 // powers of two from L = 1024 as before.
+// Below 16 tiles a workgroup's tiles cost less than the merge: one split (L = 192
+// and 240 with 1 pair 4.8 / 6.4 (3 splits), 5.4 / 6.8, with 8 5.1 / 5.9, 5.6 / 6.2,
+// with 128 5.9 / 6.4 (2 splits); at 16 tiles and 12 pairs 5.4 / 6.6).
 // A split holds at least 4 tiles, 6 above 8 splits and 8 above 32; and, but
 // for the count of a workgroup per CU, the records fit the scratch array of
 // db_f4_splitkv_noalloc whatever the head group is.
@@ -804,20 +807,25 @@ int f4_choose_splits(int B, int Hkv, int L, int cu_count) {
   const Tuning defaults;
   if (t.f4_blocks_per_cu != defaults.f4_blocks_per_cu || t.f4_min_tiles != defaults.f4_min_tiles)
     return S0;
+  if (ntiles < 16) return S0;
   if (S0 > 1 && (long)pairs * S0 == cu_count && ntiles % S0 == 0) return S0;  // one full round
   auto cost = [&](unsigned S) {
     const unsigned tps = (ntiles + S - 1) / S;
     const unsigned used = (ntiles + tps - 1) / tps;
     const unsigned rounds = (unsigned)(((size_t)pairs * used + cu_count - 1) / cu_count);
+    const float few = pairs % 8 == 0 ? 1.5f : 3.2f, launch = pairs % 8 == 0 ? 0.0f : 0.3f;
     const float merge = used == 1                  ? 0.0f
-                        : used <= kMergeChunk      ? 1.5f
-                        : used <= 16 || used >= 32 ? 2.9f
-                                                   : 3.5f;
+                        : used <= kMergeChunk      ? few
+                        : used <= 16 || used >= 32 ? 2.9f + launch
+                                                   : 3.5f + launch;
     return 0.3f * (float)rounds * tps + 1.6f * (float)(rounds - 1) + merge;
   };
   const size_t per_split = 8 * (sizeof(float2) + kD * sizeof(float));  // 8 heads per pair
   int best = S0;
-  float least = cost(S0) * 0.95f;  // a change has to be worth 5%
+  // A change has to be worth 5%, and 15% where the pairs alone fill the chip:
+  // their rounds overlap (48 x 8 pairs at L = 496 in 1.5 rounds 20.0, in 3 with 2
+  // splits 23.8; 100 x 3 pairs at L = 1024 36.0, with 3 splits 31.1).
+  float least = cost(S0) * (pairs > cu_count ? 0.85f : 0.95f);
   auto consider = [&](int S) {
     if (S < 1 || S > 256 || S > ntiles) return;
     if (S > 1 && ntiles < S * (S <= kMergeChunk ? 4 : S <= 32 ? 6 : 8)) return;

@@ -44,6 +44,19 @@ def test_default_splits_fill_their_rounds(lib):
         assert pairs * used >= 0.75 * rounds * CUS, (pairs, used)
 
 
+def test_contexts_that_a_merge_costs_more_than(lib):
+    """Below 16 tiles one split, whatever the batch; one where the pairs alone
+    fill the chip and shorter rounds hardly shorten the whole; and no fewer splits
+    for a merge of eight where that takes a launch of its own."""
+    for pairs in (1, 2, 3, 5, 8, 12, 16, 40, 64, 96, 128, 200, 300, 512):
+        for L in (1, 64, 128, 177, 192, 208, 239, 240):
+            assert lib.db_f4_default_splits(pairs, 1, L, CUS) == 1, (pairs, L)
+    assert lib.db_f4_default_splits(75, 4, 448, CUS) == 1
+    assert lib.db_f4_default_splits(48, 8, 496, CUS) == 1
+    assert lib.db_f4_default_splits(3, 4, 1400, CUS) >= 11
+    assert lib.db_f4_default_splits(1, 8, 300, CUS) > 1
+
+
 def test_tuned_split_targets_keep_their_rule(lib):
     """Either knob away from its default: a workgroup per CU (times
     f4_blocks_per_cu), no fewer tiles per split than f4_min_tiles."""
