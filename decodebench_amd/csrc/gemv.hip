@@ -84,7 +84,12 @@ bool tile_barred(GemvMode mode, int B, int K, int N) {
 //    (fp16 39.1 / 39.0 and 40.0 / 39.1 at 12 and 16, e4m3 [11008, 4096] 20.5 /
 //    19.2 and 20.2 / 18.9; fp16 at 32 and 64, where the passes read the weights
 //    again, 46.7 / 40.9 and 91.0 / 41.1, e4m3 61.9 / 29.4); with the RMSNorm
-//    from 17 (e4m3 [8192, 2048] at 16 rows 9.5 / 10.4, fp16 14.3 / 15.0).
+//    from 17 (e4m3 [8192, 2048] at 16 rows 9.5 / 10.4, fp16 14.3 / 15.0).  Not,
+//    without the norm and above 32 rows, where the outputs are so few that all
+//    passes fit on the CUs at once and share each weight line in an XCD's L2 (e4m3
+//    [501, 4096] at 38 rows 8.2 / 9.0, [64, 2048] at 50 5.5 / 6.9, at 22 8.1 / 7.1;
+//    fp16 at K = 4096 above 48).  With it the passes are faster there too (e4m3 [443,
+//    4096] at 50 rows 6.7 / 13.0), but form fp16(x gamma) whatever its range.
 //  * F1 there: registers hold the activations up to 16 rows (fp16 [6144,
 //    4096] 11.3 / 11.5 at 4); above, more than a tile per CU (fp16 at 24 and 64
 //    rows 18.6 / 14.2, 29.9 / 19.9, e4m3 11.7 / 11.5, 17.3 / 14.3), and one tile
@@ -102,7 +107,7 @@ bool tile_barred(GemvMode mode, int B, int K, int N) {
 //    at 16 rows 28.0 / 25.2, e4m3 at 8 and 64 rows 16.0 / 14.8, 33.4 / 26.7;
 //    [1024, 8192] 7.3 / 8.4 stays, up to 64 rows ([1024, 14336] fp16 at 64 and 65
 //    21.3 / 21.5, 27.4 / 21.1; e4m3 [4096, 14336] at 128 64.0 / 36.2).
-bool tile_gemv(GemvMode mode, bool fp8, int B, int K, int N) {
+bool tile_gemv(GemvMode mode, bool fp8, int B, int K, int N, int cu_count) {
   const Tuning& t = tuning();
   if (t.gemv_tile == 1) return true;
   if (tile_barred(mode, B, K, N)) return false;
@@ -113,8 +118,10 @@ bool tile_gemv(GemvMode mode, bool fp8, int B, int K, int N) {
     return B >= 9 || weights >= (B <= 4 ? 10000000 : 4000000);
   }
   if (pair) {
-    const int from = mode == kGemvSwiGLU ? 12 : 17;
-    return B >= (t.gemv_pair_min_batch > 0 ? t.gemv_pair_min_batch : from);
+    if (t.gemv_pair_min_batch > 0) return B >= t.gemv_pair_min_batch;
+    if (mode == kGemvRmsNormSwiGLU) return B >= 17;
+    const bool one_round = (long)((N + 7) / 8) * ((B + 15) / 16) <= cu_count;
+    return B >= 12 && !(one_round && B > (!fp8 && K == 4096 ? 48 : 32));
   }
   const bool one_tile = N <= 4096;
   if (K > 4096) return N > 2048 || B > 64;
@@ -166,7 +173,7 @@ int tile_splits(GemvMode mode, bool fp8, int B, int K, int N, int cu_count) {
   const int rows = min(B, 8 * tile_groups(B, passes));
   const float x_kb = (float)rows * (float)K * (2.0f / 1024.0f);
   if (B < 9 || K < 3072 || x_kb < 250.0f) return 1;
-  if (K <= 4096 && !tile_gemv(mode, fp8, B, K, N)) return 1;
+  if (K <= 4096 && !tile_gemv(mode, fp8, B, K, N, cu_count)) return 1;
   const int t3 = tiles(3, passes), t4 = tiles(4, passes);
   const int S = t4 > 4 && t3 > 0 && t3 <= 4 ? 3 : 4;
   const int t = S == 3 ? t3 : t4;
@@ -223,7 +230,7 @@ hipError_t launch_gemv(GemvMode mode, const void* x, const void* gamma,
   if (B >= (forced_min > 0 ? forced_min : 2)) {
     int splits = ws ? tile_splits(mode, w.fp8, B, K, N, cu_count) : 1;
     if (gemv_tile_workspace_bytes(mode, splits, B, N) > ws_bytes) splits = 1;
-    if (splits > 1 || tile_gemv(mode, w.fp8, B, K, N))
+    if (splits > 1 || tile_gemv(mode, w.fp8, B, K, N, cu_count))
       return launch_gemv_tile(mode, x, gamma, w, y, B, K, N, eps, cu_count, splits, ws, stream);
   }
   if (B >= mfma_min && gemv_mfma_supported(mode, B, K, N))

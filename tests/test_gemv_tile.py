@@ -394,3 +394,31 @@ def test_split_call_without_room_for_its_workspace_takes_one_launch(monkeypatch)
         finally:
             torch.cuda.set_per_process_memory_fraction(1.0)
         assert torch.equal(y, ref)
+
+
+# Both sides of the lines at which the gate/up pair leaves the 16-row passes:
+# 256 workgroups of 8 outputs and 16 rows, and the batch.
+@pytest.mark.parametrize("mode,dtype,B,K,N,tile", [
+    ("f2n", "fp8", 17, 4096, 1024, True), ("f2", "f16", 49, 2048, 512, False),
+    ("f2", "f16", 49, 2048, 513, True),
+    ("f2", "fp8", 32, 2048, 680, True), ("f2", "fp8", 33, 2048, 680, False),
+    ("f2", "f16", 48, 4096, 512, True), ("f2", "f16", 49, 4096, 512, False),
+])
+def test_pair_of_few_outputs_keeps_its_passes(mode, dtype, B, K, N, tile):
+    print(f"[tile-few] {mode} {dtype} B={B} K={K} N={N}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(B * 7919 + K + N)
+    x = _randn(gen, B, K)
+    g = _randn(gen, K, std=0.1, mean=1.0)
+    W, s, W64 = _weights(gen, 2, N, K, dtype)
+    ops.tune("gemv_splits", 1)  # one launch, as with a given output
+    try:
+        got = {}
+        for knob in (0, 1, 2):
+            ops.tune("gemv_tile", knob)
+            got[knob] = _call(mode, x, g, W, s)
+        assert torch.equal(got[0], got[1 if tile else 2])
+        assert not torch.equal(got[1], got[2])
+        ops.tune("gemv_tile", 0)
+        _check(mode, x, g, W, s, W64)
+    finally:
+        ops.tune("gemv_splits", 0)
