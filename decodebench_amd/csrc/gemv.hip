@@ -78,7 +78,14 @@ bool tile_barred(GemvMode mode, int B, int K, int N) {
 //    rows 15.2 / 12.8 and 33.2 / 12.9.  It stays ahead where one pass does
 //    and the weights are few, so that the tile kernel's LDS staging and
 //    reduction show: [1024, 3072] at 4 rows 4.7 / 5.0, [2048, 1536] at 2
-//    rows 4.1 / 4.7 (2 rows of [8192, 8192] 24.3 / 23.5, F1 27.0 / 23.8).
+//    rows 4.1 / 4.7 (2 rows of [8192, 8192] 24.3 / 23.5, F1 27.0 / 23.8);
+//    fp16 without the norm (which the tile kernel rounds once less) also where 2 rows
+//    meet weight rows that are no whole 128-byte lines, which blocks of one line
+//    read twice ([14080, 3984] 19.1 / 24.7, gate/up [4465, 12624] 43.1 / 49.6), and
+//    for long rows of so few outputs that fewer than 256 workgroups of 4 own any
+//    ([640, 11008] at 8 rows 10.2 / 11.1, gate/up [381, 14336] at 6 11.4 / 13.9,
+//    [128, 11008] at 11 9.5 / 10.9), but not gate/up of more than 512 outputs
+//    ([635, 11008] at 5 rows 0.68 of the VALU kernel's time).
 //  * The gate/up pair at K = 2048 and 4096: 16-row passes to 11 rows ([14336,
 //    4096] fp16 38.2 / 38.8 at 4, e4m3 21.3 / 22.6), the tile kernel from 12
 //    (fp16 39.1 / 39.0 and 40.0 / 39.1 at 12 and 16, e4m3 [11008, 4096] 20.5 /
@@ -114,7 +121,11 @@ bool tile_gemv(GemvMode mode, bool fp8, int B, int K, int N, int cu_count) {
   const bool pair = gemv_is_swiglu(mode);
   const long weights = (long)N * K * (pair ? 2 : 1);
   if (!gemv_mfma_supported(mode, B, K, N)) {
-    if (B == 2) return weights >= 40000000;
+    const bool plain_f16 = !fp8 && !gemv_has_norm(mode);
+    if (B == 2) return weights >= 40000000 && !(plain_f16 && K % 64 != 0);
+    if (plain_f16 && K >= 6144 && N <= (pair ? 512 : 1023) &&
+        B <= (K > 10000 && N <= 256 ? 16 : 8))
+      return false;
     return B >= 9 || weights >= (B <= 4 ? 10000000 : 4000000);
   }
   if (pair) {

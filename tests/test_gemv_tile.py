@@ -396,6 +396,37 @@ def test_split_call_without_room_for_its_workspace_takes_one_launch(monkeypatch)
         assert torch.equal(y, ref)
 
 
+# Widths of no other MFMA kernel: both sides of the lines at which fp16 without
+# the norm stays on the VALU kernel, by row alignment (2 rows) and by outputs,
+# length and batch.
+@pytest.mark.parametrize("mode,dtype,B,K,N,tile", [
+    ("gemv", "f16", 2, 5136, 8001, False), ("gemv", "f16", 2, 5184, 8001, True),
+    ("gemv", "fp8", 2, 5136, 8001, True), ("f2n", "f16", 2, 3088, 8001, True),
+    ("gemv", "f16", 8, 11008, 1023, False), ("gemv", "f16", 8, 11008, 1024, True),
+    ("f2", "f16", 7, 6160, 512, False), ("f2", "f16", 7, 6160, 513, True),
+    ("gemv", "f16", 9, 6208, 1000, True), ("gemv", "f16", 16, 10112, 256, False),
+    ("gemv", "f16", 17, 10112, 256, True), ("f1", "f16", 8, 11008, 512, True),
+])
+def test_fp16_calls_that_stay_on_the_valu_kernel(mode, dtype, B, K, N, tile):
+    print(f"[tile-valu] {mode} {dtype} B={B} K={K} N={N}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(B * 7919 + K + N)
+    x = _randn(gen, B, K)
+    g = _randn(gen, K, std=0.1, mean=1.0)
+    W, s, W64 = _weights(gen, 2 if mode in ("f2", "f2n") else 1, N, K, dtype)
+    ops.tune("gemv_splits", 1)
+    try:
+        got = {}
+        for knob in (0, 1, 2):
+            ops.tune("gemv_tile", knob)
+            got[knob] = _call(mode, x, g, W, s)
+        assert torch.equal(got[0], got[1 if tile else 2])
+        assert not torch.equal(got[1], got[2])
+        ops.tune("gemv_tile", 0)
+        _check(mode, x, g, W, s, W64)
+    finally:
+        ops.tune("gemv_splits", 0)
+
+
 # Both sides of the lines at which the gate/up pair leaves the 16-row passes:
 # 256 workgroups of 8 outputs and 16 rows, and the batch.
 @pytest.mark.parametrize("mode,dtype,B,K,N,tile", [
