@@ -147,9 +147,11 @@ bool tile_gemv(GemvMode mode, bool fp8, int B, int K, int N, int cu_count) {
 // its share of the weights, fills its L1: 14336 columns of 64 rows are 1.8 MB
 // beside 0.45 MB of fp16 weights at N = 4096.  S workgroups with S times the
 // outputs and 1 / S of the columns read x / S each.  They pay for it with S
-// partial sums per output and a second launch, about 1.5 us and 0.7 us per
+// partial sums per output and a second launch, about 2 us and 0.7 us per
 // tile (1.4 for the pair) against the 52 GB/s at which a CU reads x between
-// weights.  Measured on MI355X (us, one launch / 4 splits): fp16 [4096, 14336] at
+// weights, and against what one launch reads, whose two passes side by side may
+// have halved x already (e4m3 [2432, 3072] at 49 rows 7.7 / 10.2, F1 fp16 [1280,
+// 3072] at 51 8.0 / 10.3).  Measured on MI355X (us, one launch / 4 splits): fp16 [4096, 14336] at
 // 12, 24 and 64 rows 23.2 / 23.1, 30.3 / 24.2, 42.7 / 28.7, e4m3 at 64 26.7 /
 // 21.6; [4096, 11008] at 12 and 41 rows 18.7 / 19.0, 26.0 / 20.3; [4096, 4096]
 // at 24 and 64 10.5 / 11.2, 13.3 / 12.8; pair [2048, 8192] at 24 and 64 17.3 /
@@ -184,14 +186,17 @@ int tile_splits(GemvMode mode, bool fp8, int B, int K, int N, int cu_count) {
   const int rows = min(B, 8 * tile_groups(B, passes));
   const float x_kb = (float)rows * (float)K * (2.0f / 1024.0f);
   if (B < 9 || K < 3072 || x_kb < 250.0f) return 1;
-  if (K <= 4096 && !tile_gemv(mode, fp8, B, K, N, cu_count)) return 1;
+  const bool tile = tile_gemv(mode, fp8, B, K, N, cu_count);
+  if (K <= 4096 && !tile) return 1;
   const int t3 = tiles(3, passes), t4 = tiles(4, passes);
   const int S = t4 > 4 && t3 > 0 && t3 <= 4 ? 3 : 4;
   const int t = S == 3 ? t3 : t4;
   if (t == 0 || (passes == 1 && t > 4)) return 1;
   const float per_tile = t > 4 ? 1.1f : pair ? 1.4f : 0.7f;
-  const float gain = x_kb * (1.0f - 1.0f / (float)S) / 52.0f;
-  return gain > 2.0f + per_tile * (float)t ? S : 1;
+  const float saved = tile ? tile_plan(mode, fp8, B, K, N, cu_count, 1).read_kb -
+                                 tile_plan(mode, fp8, B, K, N, cu_count, S).read_kb
+                           : x_kb * (1.0f - 1.0f / (float)S);
+  return saved / 52.0f > 2.0f + per_tile * (float)t ? S : 1;
 }
 
 }  // namespace

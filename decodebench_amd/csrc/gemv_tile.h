@@ -102,6 +102,16 @@ constexpr int tile_depth(int t, int nxg, bool fp8, bool norm) {
   return 4 * d * loads + other > (norm ? 250 : 290) ? 1 : d;
 }
 
+// How launch_gemv_tile runs a call (gemv_tile.hip).
+struct TilePlan {
+  int passes;     // of the batch, side by side
+  int groups;     // of 8 batch rows per workgroup
+  int tiles;      // of 16 weight rows per workgroup
+  int rows;       // outputs per workgroup
+  float read_kb;  // weights and activations that a CU reads
+};
+TilePlan tile_plan(GemvMode mode, bool fp8, int B, int K, int N, int cu_count, int splits);
+
 // Kernel choice per weight type and matrix count (each defined in its own
 // translation unit).
 TileFn gemv_tile_pick_f16(bool norm, int t, int nxg);

@@ -48,6 +48,50 @@ size_t gemv_tile_workspace_bytes(GemvMode mode, int splits, int B, int N) {
                            (size_t)splits * B * sizeof(float);
 }
 
+// Passes of up to 64 batch rows, side by side on cu_count / passes workgroups
+// each, so that the passes of a row range share an XCD's L2 copy of its
+// weights.  Twice as many passes halve the x a CU reads and double its
+// weights (from L2 for the second); one matrix takes them where the sum is no
+// larger and the tiles per workgroup stay at 3 (at 4 where it falls by a
+// fifth).  Measured on MI355X (us, one pass / two): F1 [6144, 4096] fp16 at 48
+// and 64 rows 18.9 / 17.9, 20.0 / 17.7, e4m3 at 32 and 64 11.6 / 10.3, 17.2 /
+// 13.7; e4m3 F1 [7168, 5120] at 64 20.6 / 18.6, but fp16 27.7 / 29.2.
+TilePlan tile_plan(GemvMode mode, bool fp8, int B, int K, int N, int cu_count, int splits) {
+  const bool pair = gemv_is_swiglu(mode);
+  const int per = pair ? 8 : 16;
+  auto tiles = [&](int passes, int* rows) {
+    // Outputs per workgroup: an even share of a workgroup per CU (of several
+    // rounds of them where a share would be more than 8 tiles).
+    const int slots = max(8, cu_count / passes / splits / 8 * 8);
+    const int rounds = (N + slots * per * kTileMaxTiles - 1) / (slots * per * kTileMaxTiles);
+    *rows = ((N + slots * rounds - 1) / (slots * rounds) + 3) / 4 * 4;
+    return (*rows + per - 1) / per;
+  };
+  TilePlan p;
+  p.passes = tile_passes(B);
+  p.tiles = tiles(p.passes, &p.rows);
+  if (!pair && splits == 1 && B >= 17 * p.passes) {
+    const double weights = (double)N * K * (fp8 ? 1 : 2) / cu_count;
+    const double acts = 2.0 * B * K;
+    auto read = [&](int passes) { return weights * passes + acts / passes; };
+    int rows = 0;
+    const int t2 = tiles(2 * p.passes, &rows);
+    const double ratio = read(2 * p.passes) / read(p.passes);
+    if ((t2 <= 3 && ratio <= 1.0) || (t2 <= 4 && ratio <= 0.8)) {
+      p.passes *= 2;
+      p.tiles = t2;
+      p.rows = rows;
+    }
+  }
+  p.groups = tile_groups(B, p.passes);
+  const long wgs = (long)((N + p.rows - 1) / p.rows) * p.passes * splits;
+  const float row_kb = (float)K / (float)splits / 1024.0f;  // of one byte per column
+  p.read_kb = (float)((wgs + cu_count - 1) / cu_count) * row_kb *
+              ((float)p.rows * (pair ? 2.0f : 1.0f) * (fp8 ? 1.0f : 2.0f) +
+               2.0f * (float)min(B, 8 * p.groups));
+  return p;
+}
+
 hipError_t launch_gemv_tile(GemvMode mode, const void* x, const void* gamma, const GemvWeights& w,
                             void* y, int B, int K, int N, float eps, int cu_count, int splits,
                             void* ws, hipStream_t stream) {
@@ -68,41 +112,11 @@ hipError_t launch_gemv_tile(GemvMode mode, const void* x, const void* gamma, con
   a.part = static_cast<f4*>(ws);
   a.ssq = ws ? reinterpret_cast<float*>(static_cast<char*>(ws) + part_bytes(splits, pair, B, N))
              : nullptr;
-  // Passes of up to 64 batch rows, side by side on cu_count / passes workgroups
-  // each, so that the passes of a row range share an XCD's L2 copy of its
-  // weights.  Twice as many passes halve the x a CU reads and double its
-  // weights (from L2 for the second); one matrix takes them where the sum is no
-  // larger and the tiles per workgroup stay at 3 (at 4 where it falls by a
-  // fifth).  Measured on MI355X (us, one pass / two): F1 [6144, 4096] fp16 at 48
-  // and 64 rows 18.9 / 17.9, 20.0 / 17.7, e4m3 at 32 and 64 11.6 / 10.3, 17.2 /
-  // 13.7; e4m3 F1 [7168, 5120] at 64 20.6 / 18.6, but fp16 27.7 / 29.2.
-  const int per = pair ? 8 : 16;
-  auto tiles = [&](int passes, int* rows) {
-    // Outputs per workgroup: an even share of a workgroup per CU (of several
-    // rounds of them where a share would be more than 8 tiles).
-    const int slots = max(8, cu_count / passes / splits / 8 * 8);
-    const int rounds = (N + slots * per * kTileMaxTiles - 1) / (slots * per * kTileMaxTiles);
-    *rows = ((N + slots * rounds - 1) / (slots * rounds) + 3) / 4 * 4;
-    return (*rows + per - 1) / per;
-  };
-  int passes = tile_passes(B);
-  int t = tiles(passes, &a.rows);
-  if (!pair && splits == 1 && B >= 17 * passes) {
-    const double weights = (double)N * K * (w.fp8 ? 1 : 2) / cu_count;
-    const double acts = 2.0 * B * K;
-    auto read = [&](int p) { return weights * p + acts / p; };
-    int rows = 0;
-    const int t2 = tiles(2 * passes, &rows);
-    const double ratio = read(2 * passes) / read(passes);
-    if ((t2 <= 3 && ratio <= 1.0) || (t2 <= 4 && ratio <= 0.8)) {
-      passes *= 2;
-      t = t2;
-      a.rows = rows;
-    }
-  }
-  const int nxg = tile_groups(B, passes);
+  const TilePlan p = tile_plan(mode, w.fp8, B, K, N, cu_count, splits);
+  a.rows = p.rows;
+  const int t = p.tiles, nxg = p.groups;
   int grid = (N + a.rows - 1) / a.rows;
-  if (passes > 1) grid = (grid + 7) / 8 * 8;
+  if (p.passes > 1) grid = (grid + 7) / 8 * 8;
   const TileFn fn = w.fp8 ? (pair ? gemv_tile_pick_fp8_pair : gemv_tile_pick_fp8)(norm, t, nxg)
                           : (pair ? gemv_tile_pick_f16_pair : gemv_tile_pick_f16)(norm, t, nxg);
   const int wv = tile_waves(t);

@@ -347,14 +347,17 @@ def test_split_workspace_is_bounded_at_any_batch():
 
 
 # More rows than a pass: splits of one round of workgroups, shapes that would
-# take two rounds (no splits), and long rows that no longer split.
+# take two rounds (no splits), and long rows that no longer split.  Up to one:
+# two passes side by side that read as little of x (no splits).
 @pytest.mark.parametrize("mode,dtype,B,K,N,split", [
+    ("gemv", "fp8", 49, 3072, 2432, False), ("f1", "f16", 51, 3072, 1280, False),
+    ("gemv", "f16", 41, 11008, 4096, True), ("gemv", "fp8", 28, 6144, 1408, True),
     ("gemv", "f16", 65, 11008, 2050, True), ("gemv", "fp8", 129, 14336, 1024, True),
     ("f1", "f16", 100, 8192, 2047, True), ("f2n", "f16", 130, 8192, 1021, True),
     ("gemv", "f16", 65, 4096, 4096, False), ("gemv", "fp8", 200, 8192, 4095, False),
     ("f2", "f16", 129, 8192, 2048, False), ("gemv", "f16", 257, 6144, 2040, False),
 ])
-def test_automatic_splits_above_one_pass(mode, dtype, B, K, N, split):
+def test_automatic_splits(mode, dtype, B, K, N, split):
     print(f"[tile-rows] {mode} {dtype} B={B} K={K} N={N}", flush=True)
     lib = ops.load_library()
     ops.tune("gemv_tile", 0)
