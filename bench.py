@@ -2,7 +2,8 @@
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--quick]
 
-Prints ONE JSON line.  The headline workload is the benchmark's config 2 at batch 1:
+Prints ONE JSON line, short enough to be whole in the last 8000 characters of a
+log; ``--full FILE`` writes the whole record.  The headline workload is the benchmark's config 2 at batch 1:
 F2 = gate/up GEMV + SwiGLU, x[1,4096] fp16, Wg/Wu[14336,4096] fp16 ~N(0,0.02).
 A step is one fused launch over a fresh weight replica; the replicas rotate
 through a working set larger than twice the on-die caches (8 x 4 MB L2 plus
@@ -23,8 +24,9 @@ the 256 MB Infinity Cache), so every step streams its weights from HBM.
   decomposition  Sequence.profile of the unfused torch stages (stream and
                  graph) against the fused kernels: Delta_launch and B, for
                  F1, F2, F4 and the decode layer (fp16 and fp8 weights),
-                 with the per-trial samples and a fused-vs-unfused output
-                 check that decodebench_amd.validate reads
+                 with a fused-vs-unfused output check and (in the whole
+                 record) the per-trial samples, which
+                 decodebench_amd.validate reads
   cpu_baseline   the torch CPU restatement of the reference stages
                  (oracle/stages.py) on this host's cores: F2 at full size
                  (the headline), with F1 (config 1) and F4 (L = 8192) rows
@@ -68,6 +70,9 @@ def parse_args(argv=None):
                          "decomposition and the CPU baseline")
     ap.add_argument("--cpu-seconds", type=float, default=12.0,
                     help="bound on the CPU baseline sample")
+    ap.add_argument("--full", metavar="FILE",
+                    help="also write the whole record (every row's bytes and shape, the "
+                         "decomposition's samples) to FILE as JSON")
     ap.add_argument("--trials", type=int, default=30,
                     help="trials per variant in the decomposition (the validation report "
                          "needs >= 30)")
@@ -637,6 +642,34 @@ def cpu_baseline(seconds: float) -> dict:
     return out
 
 
+def short_record(out: dict) -> dict:
+    """The record with its tables cut to the figures, for the printed line."""
+    short = {k: v for k, v in out.items() if k not in (
+        "kernels", "f4_two_launch_parts", "roofline_by_kernel", "decomposition", "cpu_baseline")}
+    if "kernels" in out:
+        short["kernels_us_gbs"] = {k: [round(v["us"], 2), round(v["GB/s"])]
+                                   for k, v in out["kernels"].items()}
+    if "roofline_by_kernel" in out:
+        short["roofline_by_kernel"] = {
+            name: {k: row[k] for k in ("bound", "achieved", "peak", "unit", "frac", "us", "traffic",
+                                       "rocprof_us") if row.get(k) is not None}
+            for name, row in out["roofline_by_kernel"].items()}
+    if "decomposition" in out:
+        short["decomposition"] = {
+            name: {**{k: row[k] for k in ("t_stream_us", "t_graph_us", "t_fused_us",
+                                          "t_fused_graph_us", "delta_launch_us", "B_us",
+                                          "residual_graph_us", "bound")},
+                   "fused_check": row["fused_check"]["ok"]}
+            for name, row in out["decomposition"].items()}
+    if "cpu_baseline" in out:
+        cb = out["cpu_baseline"]
+        short["cpu_baseline"] = {
+            **{k: cb[k] for k in ("value", "unit", "cores", "kind", "sample")},
+            "us_per_call": {"f2_cfg2": cb["us_per_call"],
+                            **{k: v["us_per_call"] for k, v in cb["rows"].items()}}}
+    return short
+
+
 # -------------------------------------------------------------------- main
 def main(argv=None) -> int:
     args = parse_args(argv)
@@ -683,7 +716,7 @@ def main(argv=None) -> int:
         "scaling": "weak", "vs_baseline": None, "dtype": "f16",
         "data": "synthetic (seeded torch.Generator(42), fp32 -> fp16)",
         "config": {"workload": "F2 gate/up GEMV + SwiGLU fused, batch 1, x[1,4096], "
-                               "Wg/Wu[14336,4096] fp16 (benchmark configs[1])",
+                               "Wg/Wu[14336,4096] fp16",
                    "batch": 1, "K": 4096, "N": 14336,
                    "weight_replicas": len(head.replicas), "device": dev_name},
         "roofline": {"bound": "hbm", "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS,
@@ -761,7 +794,10 @@ def main(argv=None) -> int:
         cb = out["cpu_baseline"]
         log(f"cpu baseline: F2 {cb['value']} GB/s on {cb['cores']} threads; "
             + "; ".join(f"{k} {v['us_per_call']} us" for k, v in cb["rows"].items()))
-    print(json.dumps(out), flush=True)
+    if args.full:
+        with open(args.full, "w") as f:
+            json.dump(out, f)
+    print(json.dumps(short_record(out)), flush=True)
     return 0
 
 

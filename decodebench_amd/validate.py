@@ -383,7 +383,7 @@ def _load_json(path: str) -> dict:
         return json.loads(text)
     except ValueError:
         pass
-    # bench.py's stdout captured with its log lines: the last JSON line
+    # a record captured with log lines around it: the last JSON line
     for line in reversed(text.strip().splitlines()):
         if line.strip().startswith("{"):
             try:
@@ -395,7 +395,7 @@ def _load_json(path: str) -> dict:
 
 def main(argv=None) -> int:
     ap = argparse.ArgumentParser(description="DecodeBench validation report (fail-closed)")
-    ap.add_argument("--bench", required=True, help="bench.py output (JSON line)")
+    ap.add_argument("--bench", required=True, help="the record bench.py --full writes")
     ap.add_argument("--traffic", required=True,
                     help="decodebench_amd.rocprof --json summary with the unfused rows")
     ap.add_argument("--kernel-trace", default=None,
