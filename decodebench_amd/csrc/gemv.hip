@@ -231,8 +231,9 @@ hipError_t launch_gemv(GemvMode mode, const void* x, const void* gamma,
                        const GemvWeights& w, void* y, int B, int K, int N, float eps,
                        int cu_count, void* ws, size_t ws_bytes, hipStream_t stream) {
   const int forced_min = tuning().gemv_mfma_min_batch;
-  // Where gemv_mfma.hip takes the width.  At 3 rows the VALU kernel would run two 2-row passes, 1.5-1.8x the MFMA
-  // time.  At 2 rows (graph back-to-back, us, VALU / MFMA) MFMA takes the
+  // From how many rows gemv_mfma.hip takes a width that it has, unless the tile
+  // kernel does.  At 3 rows the VALU kernel would run two 2-row passes, 1.5-1.8x
+  // the MFMA time.  At 2 rows (graph back-to-back, us, VALU / MFMA) MFMA takes the
   // e4m3 modes with a norm or two matrices (F1 [4096, 4096] 5.87 / 5.46,
   // F1-QKV 7.17 / 6.81, gate/up pair 22.4 / 19.2, RMSNorm -> gate/up 23.2 /
   // 19.8) and rows longer than 4096 (down projection [4096, 14336] fp16
