@@ -165,8 +165,8 @@ bool tile_gemv(GemvMode mode, bool fp8, int B, int K, int N, int cu_count) {
 // 32.5; e4m3 [1024, 14336] at 129 20.8 / 17.2), 4096 columns do not ([4096, 4096]
 // at 65 and 128 13.7 / 16.1, 15.8 / 20.1), and neither does a count whose
 // workgroups take another round ([4096, 4096] at 256 21.1 / 32.1, [5120, 5120]
-// F1 34.7 / 61.8; of 24 shapes at 129 to 1024 rows 5 lost by it, most [4096,
-// 14336] at 256 rows, 83 / 69).  That bounds the workspace to 8 MB at any batch.
+// F1 34.7 / 61.8; of 20 shapes at 129 to 1024 rows 8 lose by the line at some
+// batch, most [1024, 14336] at 1024 and [4096, 14336] at 256 rows, 83 / 69).  That bounds the workspace to 8 MB at any batch.
 int tile_splits(GemvMode mode, bool fp8, int B, int K, int N, int cu_count) {
   const bool pair = gemv_is_swiglu(mode);
   const int forced = tuning().gemv_splits;
