@@ -91,12 +91,14 @@ bool tile_barred(GemvMode mode, int B, int K, int N) {
 //    (fp16 39.1 / 39.0 and 40.0 / 39.1 at 12 and 16, e4m3 [11008, 4096] 20.5 /
 //    19.2 and 20.2 / 18.9; fp16 at 32 and 64, where the passes read the weights
 //    again, 46.7 / 40.9 and 91.0 / 41.1, e4m3 61.9 / 29.4); with the RMSNorm
-//    from 17 (e4m3 [8192, 2048] at 16 rows 9.5 / 10.4, fp16 14.3 / 15.0).  Not,
-//    without the norm and above 32 rows, where the outputs are so few that all
-//    passes fit on the CUs at once and share each weight line in an XCD's L2 (e4m3
-//    [501, 4096] at 38 rows 8.2 / 9.0, [64, 2048] at 50 5.5 / 6.9, at 22 8.1 / 7.1;
-//    fp16 at K = 4096 above 48).  With it the passes are faster there too (e4m3 [443,
-//    4096] at 50 rows 6.7 / 13.0), but form fp16(x gamma) whatever its range.
+//    from 17 (e4m3 [8192, 2048] at 16 rows 9.5 / 10.4, fp16 14.3 / 15.0).  Not
+//    where the outputs are so few that all passes fit on the CUs at once and share
+//    each weight line in an XCD's L2 (norm e4m3 [1024, 4096] at 24 rows 7.2 / 9.0,
+//    [512, 4096] at 59 7.1 / 13.5, fp16 [866, 4096] at 32 8.7 / 10.1; one row of
+//    passes more, [1280, 4096] at 20, 10.8 / 8.3); without the norm, whose sums of
+//    x^2 cost the tile kernel most of that, only above 32 rows (e4m3 [501, 4096] at
+//    38 8.2 / 9.0, [64, 2048] at 50 5.5 / 6.9, at 22 8.1 / 7.1), fp16 at K = 4096
+//    above 48.
 //  * F1 there: registers hold the activations up to 16 rows (fp16 [6144,
 //    4096] 11.3 / 11.5 at 4); above, more than a tile per CU (fp16 at 24 and 64
 //    rows 18.6 / 14.2, 29.9 / 19.9, e4m3 11.7 / 11.5, 17.3 / 14.3), and one tile
@@ -130,8 +132,8 @@ bool tile_gemv(GemvMode mode, bool fp8, int B, int K, int N, int cu_count) {
   }
   if (pair) {
     if (t.gemv_pair_min_batch > 0) return B >= t.gemv_pair_min_batch;
-    if (mode == kGemvRmsNormSwiGLU) return B >= 17;
     const bool one_round = (long)((N + 7) / 8) * ((B + 15) / 16) <= cu_count;
+    if (mode == kGemvRmsNormSwiGLU) return B >= 17 && !one_round;
     return B >= 12 && !(one_round && B > (!fp8 && K == 4096 ? 48 : 32));
   }
   const bool one_tile = N <= 4096;

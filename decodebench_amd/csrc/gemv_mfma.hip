@@ -118,7 +118,11 @@ struct MfmaArgs {
 // 8 per wave) and read back per group, so every weight tile feeds 32 rows in
 // one workgroup; the default instead runs two 16-row passes that share the
 // weights through an XCD's L2.
-template <int MODE, int KH, int BT, bool FP8, bool XB>
+// RANGE (norm modes, not XB): rows outside fp16's comfortable range are scaled.
+// Only for RMSNorm -> gate/up above 16 rows, whose other kernel (gemv_tile.h) does
+// so too.  It makes the first product wait for the statistic: F1 at 9 to 16 rows
+// would lose 0.1-0.3 us by it (e4m3 [4096, 2048] 5.0 -> 5.3 us).
+template <int MODE, int KH, int BT, bool FP8, bool XB, bool RANGE = false>
 __global__ __launch_bounds__(kThreadsM) void gemv_mfma_kernel(MfmaArgs a) {
   constexpr int NWM = gemv_is_swiglu(MODE) ? 2 : 1;
   constexpr int KW = FP8 ? KH / 2 : KH;  // 16-byte weight loads per row and slice
@@ -352,6 +356,9 @@ __global__ __launch_bounds__(kThreadsM) void gemv_mfma_kernel(MfmaArgs a) {
   __builtin_amdgcn_sched_barrier(0);
 
 
+  float unscale[BT];  // norm modes: 1 / the scale of batch row 8 bt + r8
+#pragma unroll
+  for (int bt = 0; bt < BT; ++bt) unscale[bt] = 1.0f;
   if constexpr (gemv_has_norm(MODE)) {
     // x^2 over this slice per batch row: in-lane, then over the two halves
     // (lanes 8 apart) and the 4 k-groups (lanes 16 apart).
@@ -370,6 +377,35 @@ __global__ __launch_bounds__(kThreadsM) void gemv_mfma_kernel(MfmaArgs a) {
       if ((int)threadIdx.x < a.K / 8) s_gamma[threadIdx.x] = gchunk;
       __syncthreads();
     } else {
+      if constexpr (RANGE) {
+        // The operands are fp16(x * gamma), whose range follows x's: where a
+        // row's slice has a mean square outside [2^-4, 2^4], or all of gamma's
+        // is so small that its products would be subnormal, the wave's rows are
+        // scaled by the powers of two (exact) that bring them near 1, and its
+        // sums back as they are stored.
+        constexpr float per_col = 1.0f / (64 * KH);
+        bool need = __all(lane >= 8 * KH || dot8(gchunk, gchunk, 0.0f) < 8 * 0x1p-20f);
+#pragma unroll
+        for (int bt = 0; bt < BT; ++bt) {
+          const float ms = ss[bt] * per_col;
+          need = need || (ms > 0.0f && (ms < 0x1p-4f || ms > 0x1p4f));
+        }
+        if (__any(need)) {
+#pragma unroll
+          for (int bt = 0; bt < BT; ++bt) {
+            const float ms = ss[bt] * per_col;
+            int e = ms > 0.0f ? (1 - __builtin_amdgcn_frexp_expf(ms)) >> 1 : 0;
+            e = max(-16, min(15, e));
+            const _Float16 f = (_Float16)__builtin_amdgcn_ldexpf(1.0f, e);
+            unscale[bt] = __builtin_amdgcn_ldexpf(1.0f, -e);
+#pragma unroll
+            for (int t = 0; t < KH; ++t)
+#pragma unroll
+              for (int q = 0; q < 4; ++q)
+                xr[bt][t][q] = __builtin_bit_cast(unsigned, as_h2(xr[bt][t][q]) * h2{f, f});
+          }
+        }
+      }
       // The wave's slice of gamma (chunks sbase / 8 ..), read back by the
       // wave's own lanes.
       if (lane < 8 * KH) s_gamma[wave * kWave + lane] = gchunk;
@@ -452,6 +488,7 @@ __global__ __launch_bounds__(kThreadsM) void gemv_mfma_kernel(MfmaArgs a) {
           // (g4 < 2, c16 < 8); their half-1 partners sit 40 lanes higher.
 #pragma unroll
           for (int i = 0; i < 4; ++i) acc[i] += __shfl(acc[i], lane + 40);
+          if constexpr (RANGE) acc *= unscale[bt];
           // The first partial-sum store of the workgroup: a staging area it
           // shares must have been read back by every wave (j is uniform, and
           // every workgroup consumes group 0 first, exactly once).
@@ -800,6 +837,12 @@ MfmaFn pick_xb(int kh) {
 }
 
 template <bool FP8>
+MfmaFn pick_range(int kh) {
+  return kh == 4 ? gemv_mfma_kernel<kGemvRmsNormSwiGLU, 4, 2, FP8, false, true>
+                 : gemv_mfma_kernel<kGemvRmsNormSwiGLU, 8, 2, FP8, false, true>;
+}
+
+template <bool FP8>
 MfmaFn pick_mode(GemvMode mode, int kh, int bt, bool xb) {
   if (xb) return mode == kGemvRmsNorm ? pick_xb<kGemvRmsNorm, FP8>(kh)
                                       : pick_xb<kGemvPlain, FP8>(kh);
@@ -955,7 +998,10 @@ hipError_t launch_gemv_mfma(GemvMode mode, const void* x, const void* gamma,
   const bool xb = !split_passes && nwm == 1 && B > kBatchTile && xb_bytes + part32 <= 152 * 1024;
   const int bt = xb || B >= 9 ? 2 : 1;  // batch column tiles held in registers
   const int pass = xb ? 32 : kBatchTile;
-  const MfmaFn fn = w.fp8 ? pick_mode<true>(mode, kh, bt, xb) : pick_mode<false>(mode, kh, bt, xb);
+  const bool range = mode == kGemvRmsNormSwiGLU && B > kBatchTile;
+  const MfmaFn fn = range   ? (w.fp8 ? pick_range<true>(kh) : pick_range<false>(kh))
+                    : w.fp8 ? pick_mode<true>(mode, kh, bt, xb)
+                            : pick_mode<false>(mode, kh, bt, xb);
   // The activation staging (the norm modes, and one matrix at two batch
   // tiles) without XB -- each wave's slice of the pass's rows, 16 bytes per
   // lane per row tile and k-step -- shares the partial-sum region.

@@ -46,8 +46,8 @@ extern "C" {
  *                         a multiple of 2048) on that kernel, K splits or not
  *  "gemv_pair_min_batch" (batch rows from which the gate/up pair at K = 2048
  *                         and 4096 streams its activations on 16 x 16 tiles;
- *                         0 automatic, 12, with the RMSNorm 17; few outputs
- *                         stay off it above 32 rows, without the RMSNorm)
+ *                         0 automatic, 12, with the RMSNorm 17, where the
+ *                         outputs are not few)
  *  "gemv_tile"           (batches of 2 rows and more: 1 always the streamed
  *                         16 x 16 tile kernel, 2 never, K splits included; 0
  *                         automatic)

@@ -223,6 +223,31 @@ def test_tile_norm_keeps_precision_under_a_small_gamma(std, dtype):
     assert err <= 4.5e-4, f"{err.item():.2e}"
 
 
+@pytest.mark.parametrize("dtype,B,K,N", [("f16", 17, 2048, 700), ("fp8", 24, 4096, 333),
+                                         ("f16", 49, 4096, 500), ("fp8", 64, 2048, 512)])
+def test_pair_passes_keep_precision_over_the_fp16_range(dtype, B, K, N):
+    """RMSNorm -> gate/up of few outputs above 16 rows, which the 16-row passes
+    take: x at every scale, one block unlike the others, one product of gamma
+    that leaves fp16, rows of zeros, and gamma of 2^-13."""
+    gen = torch.Generator(device="cuda").manual_seed(B + K)
+    ops.tune("gemv_tile", 0)
+    weights = _weights(gen, 2, N, K, dtype)
+    g = _randn(gen, K, std=0.1, mean=1.0)
+    for std in (2.0 ** -13, 1e-3, 0.12, 0.24, 0.26, 1.0, 3.9, 4.1, 200.0, 1.2e4):
+        print(f"[pass-range] {dtype} B={B} K={K} N={N} std={std}", flush=True)
+        x = _randn(gen, B, K).sign() * (1 + 0.5 * torch.rand(B, K, generator=gen, device="cuda"))
+        _check("f2n", (x * std).half(), g, *weights)
+    for e in (-12, 9):
+        x = _randn(gen, B, K).float()
+        x[:, K // 2:K // 2 + 256] *= 2.0 ** e
+        x[3] = 0
+        _check("f2n", x.half(), g, *weights)
+    x = _randn(gen, B, K, std=60.0)
+    x[:, 9] = 3000.0
+    _check("f2n", x, _randn(gen, K, std=1.0, mean=24.0), *weights)
+    _check("f2n", _randn(gen, B, K, std=0.3), (g.float() * 2.0 ** -13).half(), *weights)
+
+
 # K split over workgroups: counts that divide the blocks and that do not, a
 # last split of one block, outputs that no quad or tile divides, more rows
 # than a pass, every mode and weight type.
@@ -433,8 +458,9 @@ def test_fp16_calls_that_stay_on_the_valu_kernel(mode, dtype, B, K, N, tile):
 # Both sides of the lines at which the gate/up pair leaves the 16-row passes:
 # 256 workgroups of 8 outputs and 16 rows, and the batch.
 @pytest.mark.parametrize("mode,dtype,B,K,N,tile", [
-    ("f2n", "fp8", 17, 4096, 1024, True), ("f2", "f16", 49, 2048, 512, False),
-    ("f2", "f16", 49, 2048, 513, True),
+    ("f2n", "fp8", 17, 4096, 1024, False), ("f2n", "fp8", 17, 4096, 1025, True),
+    ("f2n", "f16", 49, 2048, 512, False), ("f2n", "f16", 49, 2048, 513, True),
+    ("f2", "f16", 49, 2048, 512, False), ("f2", "f16", 49, 2048, 513, True),
     ("f2", "fp8", 32, 2048, 680, True), ("f2", "fp8", 33, 2048, 680, False),
     ("f2", "f16", 48, 4096, 512, True), ("f2", "f16", 49, 4096, 512, False),
 ])
