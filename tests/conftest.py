@@ -6,6 +6,7 @@ GPU box they run against the in-tree HIP library and fail loudly if it is
 missing.
 """
 
+import gc
 import os
 import sys
 
@@ -36,3 +37,17 @@ def pytest_collection_modifyitems(config, items):
     for item in items:
         if "gpu" in item.keywords:
             item.add_marker(skip)
+
+
+@pytest.fixture(autouse=True)
+def _no_collection_while_memory_is_compared(request):
+    """The no-allocation tests compare allocated bytes before and after a call:
+    tensors that earlier tests left in reference cycles are freed before them,
+    and none in between."""
+    if request.module.__name__.split(".")[-1] != "test_zz_no_alloc":
+        yield
+        return
+    gc.collect()
+    gc.disable()
+    yield
+    gc.enable()
